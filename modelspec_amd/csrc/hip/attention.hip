@@ -5,8 +5,7 @@
 // them to the P V and dS K MFMAs without an LDS round trip. The forward is one pass over the keys
 // (online softmax) and saves each query's softmax maximum and sum; the backward recomputes P from
 // them and takes
-// d_i = sum_j P_ij dP_ij as rowsum(dO_i * O_i) from the forward's output. Shapes outside the MFMA
-// tiling run a scalar fallback (one thread per row). Semantics: interpreter.rs:1035-1119,
+// d_i = sum_j P_ij dP_ij as rowsum(dO_i * O_i) from the forward's output. Semantics: interpreter.rs:1035-1119,
 // 1298-1510 (masked keys excluded; a masked key's dK and dV rows are +0).
 #include <algorithm>
 #include <cmath>
@@ -27,177 +26,20 @@ __device__ __forceinline__ v4f mfma4(float a, float b, v4f c) { return __builtin
 }  // namespace
 
 // ---------------------------------------------------------------------------------------------
-// Scalar fallback.
-template <int D>
-__global__ __launch_bounds__(64) void k_attn_fwd_scalar(const float* __restrict__ q, const float* __restrict__ k,
-                                                 const float* __restrict__ v, const float* __restrict__ mask,
-                                                 float* __restrict__ o, int L, int S, int H, int heads, float scale) {
-  extern __shared__ float sm[];
-  float* Ks = sm;
-  float* Vs = sm + S * D;
-  float* Ms = sm + 2 * S * D;
-  const int b = blockIdx.x / heads, head = blockIdx.x % heads;
-  for (int e = threadIdx.x; e < S * D; e += blockDim.x) {
-    int j = e / D, c = e % D;
-    Ks[e] = k[(int64_t(b) * S + j) * H + head * D + c];
-    Vs[e] = v[(int64_t(b) * S + j) * H + head * D + c];
-  }
-  for (int j = threadIdx.x; j < S; j += blockDim.x) Ms[j] = mask[int64_t(b) * S + j];
-  __syncthreads();
-  const int i = blockIdx.y * blockDim.x + threadIdx.x;
-  if (i >= L) return;
-  const int64_t row = int64_t(b) * L + i;
-  float qr[D], acc[D];
-#pragma unroll
-  for (int c = 0; c < D; ++c) { qr[c] = q[row * H + head * D + c]; acc[c] = 0.0f; }
-  float mx = 0.0f;
-  bool first = true;
-  for (int j = 0; j < S; ++j) {
-    if (Ms[j] == 0.0f) continue;
-    const float* kj = Ks + j * D;
-    float sc = qr[0] * kj[0];
-#pragma unroll
-    for (int c = 1; c < D; ++c) sc = __builtin_fmaf(qr[c], kj[c], sc);
-    sc = sc * scale;
-    if (first || sc > mx) mx = sc;
-    first = false;
-  }
-  float total = 0.0f;
-  for (int j = 0; j < S; ++j) {
-    if (Ms[j] == 0.0f) continue;
-    const float* kj = Ks + j * D;
-    float sc = qr[0] * kj[0];
-#pragma unroll
-    for (int c = 1; c < D; ++c) sc = __builtin_fmaf(qr[c], kj[c], sc);
-    float e = expf(sc * scale - mx);
-    total += e;
-    const float* vj = Vs + j * D;
-#pragma unroll
-    for (int c = 0; c < D; ++c) acc[c] = __builtin_fmaf(e, vj[c], acc[c]);
-  }
-#pragma unroll
-  for (int c = 0; c < D; ++c) o[row * H + head * D + c] = acc[c] / total;
-}
-
-template <int D>
-__global__ __launch_bounds__(256) void k_attn_bwd_scalar(const float* __restrict__ q, const float* __restrict__ k,
-                                                  const float* __restrict__ v, const float* __restrict__ mask,
-                                                  const float* __restrict__ g, float* __restrict__ dq,
-                                                  float* __restrict__ dk, float* __restrict__ dv, int L, int S, int H,
-                                                  int heads, float scale) {
-  extern __shared__ float sm[];
-  float* Qs = sm;
-  float* Gs = Qs + L * D;
-  float* Ks = Gs + L * D;
-  float* Vs = Ks + S * D;
-  float* Ms = Vs + S * D;
-  float* st_m = Ms + S;
-  float* st_l = st_m + L;
-  float* st_d = st_l + L;
-  const int b = blockIdx.x / heads, head = blockIdx.x % heads;
-  for (int e = threadIdx.x; e < L * D; e += blockDim.x) {
-    int i = e / D, c = e % D;
-    Qs[e] = q[(int64_t(b) * L + i) * H + head * D + c];
-    Gs[e] = g[(int64_t(b) * L + i) * H + head * D + c];
-  }
-  for (int e = threadIdx.x; e < S * D; e += blockDim.x) {
-    int j = e / D, c = e % D;
-    Ks[e] = k[(int64_t(b) * S + j) * H + head * D + c];
-    Vs[e] = v[(int64_t(b) * S + j) * H + head * D + c];
-  }
-  for (int j = threadIdx.x; j < S; j += blockDim.x) Ms[j] = mask[int64_t(b) * S + j];
-  __syncthreads();
-  auto dot = [](const float* x, const float* y) {
-    float s = x[0] * y[0];
-#pragma unroll
-    for (int c = 1; c < D; ++c) s = __builtin_fmaf(x[c], y[c], s);
-    return s;
-  };
-  // Phase 1, per query row: softmax statistics, d = sum_j P dP, and dQ.
-  for (int i = threadIdx.x; i < L; i += blockDim.x) {
-    const float* qi = Qs + i * D;
-    const float* gi = Gs + i * D;
-    float mx = 0.0f;
-    bool first = true;
-    for (int j = 0; j < S; ++j) {
-      if (Ms[j] == 0.0f) continue;
-      float sc = dot(qi, Ks + j * D) * scale;
-      if (first || sc > mx) mx = sc;
-      first = false;
-    }
-    float total = 0.0f;
-    for (int j = 0; j < S; ++j) {
-      if (Ms[j] == 0.0f) continue;
-      total += expf(dot(qi, Ks + j * D) * scale - mx);
-    }
-    float dd = 0.0f;
-    for (int j = 0; j < S; ++j) {
-      if (Ms[j] == 0.0f) continue;
-      float p = expf(dot(qi, Ks + j * D) * scale - mx) / total;
-      dd = __builtin_fmaf(p, dot(gi, Vs + j * D), dd);
-    }
-    st_m[i] = mx;
-    st_l[i] = total;
-    st_d[i] = dd;
-    if (dq) {
-      float acc[D];
-#pragma unroll
-      for (int c = 0; c < D; ++c) acc[c] = 0.0f;
-      for (int j = 0; j < S; ++j) {
-        if (Ms[j] == 0.0f) continue;
-        float p = expf(dot(qi, Ks + j * D) * scale - mx) / total;
-        float ds = p * (dot(gi, Vs + j * D) - dd);
-        const float* kj = Ks + j * D;
-#pragma unroll
-        for (int c = 0; c < D; ++c) acc[c] = __builtin_fmaf(ds, kj[c], acc[c]);
-      }
-#pragma unroll
-      for (int c = 0; c < D; ++c) dq[(int64_t(b) * L + i) * H + head * D + c] = acc[c] * scale;
-    }
-  }
-  __syncthreads();
-  // Phase 2, per key row: dV = sum_i P g_i, dK = scale * sum_i dS q_i; a masked key stays +0.
-  for (int j = threadIdx.x; j < S; j += blockDim.x) {
-    const int64_t out = (int64_t(b) * S + j) * H + head * D;
-    const bool live = Ms[j] != 0.0f;
-    if (dv) {
-      float acc[D];
-#pragma unroll
-      for (int c = 0; c < D; ++c) acc[c] = 0.0f;
-      if (live)
-        for (int i = 0; i < L; ++i) {
-          float p = expf(dot(Qs + i * D, Ks + j * D) * scale - st_m[i]) / st_l[i];
-          const float* gi = Gs + i * D;
-#pragma unroll
-          for (int c = 0; c < D; ++c) acc[c] = __builtin_fmaf(p, gi[c], acc[c]);
-        }
-#pragma unroll
-      for (int c = 0; c < D; ++c) dv[out + c] = acc[c];
-    }
-    if (dk) {
-      float acc[D];
-#pragma unroll
-      for (int c = 0; c < D; ++c) acc[c] = 0.0f;
-      if (live)
-        for (int i = 0; i < L; ++i) {
-          const float* qi = Qs + i * D;
-          float p = expf(dot(qi, Ks + j * D) * scale - st_m[i]) / st_l[i];
-          float ds = p * (dot(Gs + i * D, Vs + j * D) - st_d[i]);
-#pragma unroll
-          for (int c = 0; c < D; ++c) acc[c] = __builtin_fmaf(ds, qi[c], acc[c]);
-        }
-#pragma unroll
-      for (int c = 0; c < D; ++c) dk[out + c] = live ? acc[c] * scale : 0.0f;
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------------------------
-// MFMA path. A block is four waves; each wave owns 16 rows of its side (queries for the forward
+// A block is four waves; each wave owns 16 rows of its side (queries for the forward
 // and dQ, keys for dK/dV) and the block streams the other side through LDS in tiles of T rows,
 // double-buffered: the next tile's global loads are in flight while the current one is in the
 // MFMAs, and one barrier a tile hands the buffers over. Row stride of every LDS tile is D + 4
 // floats: the 16 rows x 4 columns an MFMA operand read touches fall in distinct banks.
+
+// The f32 kernels take any row count; one that is no multiple of 16 leaves a partial last tile. A
+// scalar kernel (one thread a row, a head a block) took such sequences before: 2186 us backward and
+// 158 us forward a layer for 36 heads of 100 x 64, every row walking all keys serially, against
+// 18.1 and 10.2 us here. A wave's own rows past the end
+// (own_row) and a tile's (fetch_pair) repeat the last row; the streamed ones take no part: a key
+// past the end carries mask 0, a query past the end the maximum +inf, so that its probability is
+// exp(-inf) = 0. Rows past the end are not written.
+__device__ __forceinline__ int own_row(int first, int c, int rows) { return first + c < rows ? first + c : rows - 1; }
 
 // Scores of U tiles of 16 LDS rows R against the 16 columns whose operand fragments xb a lane
 // holds: acc[u][r] = sum over d of R[16 u + c][d] x[4 g + r][d], each in d order. Tiles at or past
@@ -282,7 +124,7 @@ __global__ __launch_bounds__(64 * W) void k_attn_fwd_mfma(const float* __restric
   const int half = wave % KS;
   const int i0 = blockIdx.y * (16 * W / KS) + (wave / KS) * 16;
   const bool active = i0 < L;
-  const int64_t qrow = (int64_t(b) * L + (active ? i0 : 0) + c) * H + head * D;
+  const int64_t qrow = (int64_t(b) * L + own_row(i0, c, L)) * H + head * D;
   float qb[D / 4];
 #pragma unroll
   for (int t = 0; t < D / 4; ++t) qb[t] = q[qrow + 4 * t + g];
@@ -294,7 +136,7 @@ __global__ __launch_bounds__(64 * W) void k_attn_fwd_mfma(const float* __restric
   {
     v4f kv[PT], vv[PT];
     fetch_pair<D, T, NT>(kv, vv, k + kbase, v + kbase, H, S < T ? S : T);
-    const float mv = tid < T ? mrow[tid < S ? tid : S - 1] : 0.0f;
+    const float mv = tid < T && tid < S ? mrow[tid] : 0.0f;
     put_pair<D, T, NT>(Kb, Vb, kv, vv);
     if (tid < T) Mb[tid] = mv;
   }
@@ -311,9 +153,9 @@ __global__ __launch_bounds__(64 * W) void k_attn_fwd_mfma(const float* __restric
     if (more) {
       const int s1 = s0 + T, n1 = S - s1 < T ? S - s1 : T;
       fetch_pair<D, T, NT>(kv, vv, k + kbase + int64_t(s1) * H, v + kbase + int64_t(s1) * H, H, n1);
-      if (tid < T) mv = mrow[s1 + (tid < n1 ? tid : n1 - 1)];
+      if (tid < T && tid < n1) mv = mrow[s1 + tid];
     }
-    const int nt = KS == 1 ? n / 16 : std::min(U, n / 16 - half * U);
+    const int nt = std::min(U, (n + 15) / 16 - half * U);
     if (active && nt > 0) {
       const float* Ks = Kb + j * 2 * T * DP + half * U * 16 * DP;
       const float* Vs = Vb + j * 2 * T * DP + half * U * 16 * DP;
@@ -412,11 +254,12 @@ __global__ __launch_bounds__(64 * W) void k_attn_fwd_mfma(const float* __restric
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const float row_total = __shfl(l, 4 * g + r, 64);
+    if (i0 + 4 * g + r >= L) continue;
     const int64_t orow = (int64_t(b) * L + i0 + 4 * g + r) * H + head * D;
 #pragma unroll
     for (int ct = 0; ct < D / 16; ++ct) o[orow + ct * 16 + c] = oacc[ct][r] / row_total;
   }
-  if (stats && g == 0) {
+  if (stats && g == 0 && i0 + c < L) {
     const int64_t at = (int64_t(blockIdx.x) * L + i0 + c) * 2;
     stats[at] = m;
     stats[at + 1] = l;
@@ -575,7 +418,7 @@ __device__ __forceinline__ void attn_bwd_q_body(const float* __restrict__ q, con
   const int half = wave % KS;  // KS waves share a query tile, each a share of every key tile
   const int i0 = by * (16 * W / KS) + (wave / KS) * 16;
   const bool active = i0 < L;
-  const int64_t row = (int64_t(b) * L + (active ? i0 : 0) + c) * H + head * D;
+  const int64_t row = (int64_t(b) * L + own_row(i0, c, L)) * H + head * D;
   // d_i for query i0 + c: lane group g sums columns [g D/4, (g + 1) D/4).
   float dd = 0.0f;
 #pragma unroll
@@ -587,8 +430,8 @@ __device__ __forceinline__ void attn_bwd_q_body(const float* __restrict__ q, con
   }
   dd += __shfl_xor(dd, 16, 64);
   dd += __shfl_xor(dd, 32, 64);
-  const int64_t srow = int64_t(blockIdx.x) * L + (active ? i0 : 0) + c;
-  if (dsum && active && g == 0 && half == 0) dsum[srow] = dd;
+  const int64_t srow = int64_t(blockIdx.x) * L + own_row(i0, c, L);
+  if (dsum && i0 + c < L && g == 0 && half == 0) dsum[srow] = dd;
   const float mx = stats[2 * srow], total = stats[2 * srow + 1];
   float qb[D / 4], gb[D / 4];
 #pragma unroll
@@ -601,7 +444,7 @@ __device__ __forceinline__ void attn_bwd_q_body(const float* __restrict__ q, con
   {
     v4f kv[PT], vv[PT];
     fetch_pair<D, T, NT>(kv, vv, k + kbase, v + kbase, H, S < T ? S : T);
-    const float mv = tid < T ? mrow[tid < S ? tid : S - 1] : 0.0f;
+    const float mv = tid < T && tid < S ? mrow[tid] : 0.0f;
     put_pair<D, T, NT>(Kb, Vb, kv, vv);
     if (tid < T) Mb[tid] = mv;
   }
@@ -617,9 +460,9 @@ __device__ __forceinline__ void attn_bwd_q_body(const float* __restrict__ q, con
     if (more) {
       const int s1 = s0 + T, n1 = S - s1 < T ? S - s1 : T;
       fetch_pair<D, T, NT>(kv, vv, k + kbase + int64_t(s1) * H, v + kbase + int64_t(s1) * H, H, n1);
-      if (tid < T) mv = mrow[s1 + (tid < n1 ? tid : n1 - 1)];
+      if (tid < T && tid < n1) mv = mrow[s1 + tid];
     }
-    const int nt = KS == 1 ? n / 16 : std::min(U, n / 16 - half * U);
+    const int nt = std::min(U, (n + 15) / 16 - half * U);
     if (active && nt > 0) {
       const float* Ks = Kb + j * 2 * T * DP + half * U * 16 * DP;
       const float* Vs = Vb + j * 2 * T * DP + half * U * 16 * DP;
@@ -671,6 +514,7 @@ __device__ __forceinline__ void attn_bwd_q_body(const float* __restrict__ q, con
   if (!active) return;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
+    if (i0 + 4 * g + r >= L) break;
     const int64_t orow = (int64_t(b) * L + i0 + 4 * g + r) * H + head * D;
 #pragma unroll
     for (int ct = 0; ct < D / 16; ++ct) dq[orow + ct * 16 + c] = acc[ct][r] * scale;
@@ -709,8 +553,8 @@ __device__ __forceinline__ void attn_bwd_kv_body(const float* __restrict__ q, co
   const int half = wave % KS;  // KS waves share a key tile, each a share of every query tile
   const int j0 = by * (16 * W / KS) + (wave / KS) * 16;
   const bool active = j0 < S;
-  const int64_t krow = (int64_t(b) * S + (active ? j0 : 0) + c) * H + head * D;
-  const bool live = mask[int64_t(b) * S + (active ? j0 : 0) + c] != 0.0f;
+  const int64_t krow = (int64_t(b) * S + own_row(j0, c, S)) * H + head * D;
+  const bool live = mask[int64_t(b) * S + own_row(j0, c, S)] != 0.0f;
   float kb[D / 4], vb[D / 4];
 #pragma unroll
   for (int t = 0; t < D / 4; ++t) { kb[t] = k[krow + 4 * t + g]; vb[t] = v[krow + 4 * t + g]; }
@@ -728,7 +572,7 @@ __device__ __forceinline__ void attn_bwd_kv_body(const float* __restrict__ q, co
   auto fetch_stats = [&](float (&e)[2 + PD], int l0, int n) {
     if (tid < T) {
       const int64_t at = sbase + l0 + (tid < n ? tid : n - 1);
-      e[0] = stats[2 * at];
+      e[0] = tid < n ? stats[2 * at] : INFINITY;
       e[1] = stats[2 * at + 1];
     }
 #pragma unroll
@@ -785,7 +629,7 @@ __device__ __forceinline__ void attn_bwd_kv_body(const float* __restrict__ q, co
       fetch_pair<D, T, NT>(qv, gv, q + qbase + int64_t(l1) * H, go + qbase + int64_t(l1) * H, H, n1);
       fetch_stats(e, l1, n1);
     }
-    const int nt = KS == 1 ? n / 16 : std::min(U, n / 16 - half * U);
+    const int nt = std::min(U, (n + 15) / 16 - half * U);
     if (active && nt > 0) {
       const float* Qs = Qb + j * 2 * T * DP + half * U * 16 * DP;
       const float* Gs = Gb + j * 2 * T * DP + half * U * 16 * DP;
@@ -849,6 +693,7 @@ __device__ __forceinline__ void attn_bwd_kv_body(const float* __restrict__ q, co
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int jj = j0 + 4 * g + r;
+    if (jj >= S) break;
     const bool keep = mask[int64_t(b) * S + jj] != 0.0f;
     const int64_t orow = (int64_t(b) * S + jj) * H + head * D;
 #pragma unroll
@@ -1281,8 +1126,13 @@ __global__ __launch_bounds__(64 * W) void k_attn_bwd_kv_h16(const float* __restr
 
 // ---------------------------------------------------------------------------------------------
 namespace {
-size_t scalar_fwd_lds(int64_t S, int64_t d) { return size_t((2 * S * d + S) * 4); }
-size_t scalar_bwd_lds(int64_t L, int64_t S, int64_t d) { return size_t((2 * L * d + 2 * S * d + S + 3 * L) * 4); }
+// Row counts that are no multiple of 16 are taken while a head's operands stay within one block's
+// LDS as plain f32 rows (S of at most 157 for 64-wide heads): the declared limit of such sequences.
+bool whole_tiles(int64_t L, int64_t S) { return L % 16 == 0 && S % 16 == 0; }
+bool fwd_fits(int64_t L, int64_t S, int64_t d) { return whole_tiles(L, S) || size_t(2 * S * d + S) * 4 <= kLdsMax; }
+bool bwd_fits(int64_t L, int64_t S, int64_t d) {
+  return whole_tiles(L, S) || size_t(2 * L * d + 2 * S * d + S + 3 * L) * 4 <= kLdsMax;
+}
 bool head_ok(int64_t d) { return d == 16 || d == 32 || d == 64 || d == 128; }
 // The streaming shape, from measured MI355X timings: problems of 4096 or more 16-row wave tiles
 // (BERT-base: 12288) take blocks of four waves and tiles of 32 rows (35 KB of LDS a block at
@@ -1372,13 +1222,7 @@ void launch_bwd(hipStream_t s, dim3 grid, unsigned qy, bool one, const float* q,
   }
 }  // namespace
 
-bool attention_mfma(int64_t L, int64_t S, int64_t d) {
-  return head_ok(d) && L % 16 == 0 && S % 16 == 0;
-}
-
-bool attention_fits(int64_t s, int64_t d) {
-  return head_ok(d) && s <= 65535 && (attention_mfma(s, s, d) || scalar_bwd_lds(s, s, d) <= kLdsMax);
-}
+bool attention_fits(int64_t s, int64_t d) { return head_ok(d) && s <= 65535 && bwd_fits(s, s, d); }
 
 #define MSX_BY_D(d, call)                          \
   switch (d) {                                     \
@@ -1393,34 +1237,27 @@ void attention_fwd(hipStream_t s, const float* q, const float* k, const float* v
   int64_t d = H / heads;
   if (!head_ok(d) || L > S) refuse("attention head width or query rows");
   float scale = 1.0f / sqrtf(float(d));
-  if (attention_mfma(L, S, d)) {
-    // 128 keys of 64-wide heads in f32 (BERT-tiny): the register-operand forward, four waves a
-    // 16-query tile (8.5 us a layer against 10.0 for the LDS-staged kernel; two waves 9.9, eight
-    // 9.5; the step 0.755 -> 0.751 ms). Its 16-byte loads need 16-byte aligned rows.
-    const auto al16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-    if (!h16 && d == 64 && S == 128 && H % 4 == 0 && al16(q) && al16(k) && al16(v) && al16(mask) && al16(o)) {
-      dim3 grid(unsigned(B * heads), unsigned(L / 16));
-      MSX_LAUNCH(k_attn_fwd_reg<4>, grid, dim3(256), 0, s, q, k, v, mask, o, stats, int(L), int(H), int(heads), scale);
-      return;
-    }
-    const AttnPlan plan = attn_plan(B * heads, L, S, d, h16);
-    dim3 grid(unsigned(B * heads), row_blocks(L, plan));
+  if (!fwd_fits(L, S, d)) refuse("attention shape outside the kernels' LDS budget");
+  h16 = h16 && whole_tiles(L, S);  // partial tiles stay in f32, also under mixed precision
+  // 128 keys of 64-wide heads in f32 (BERT-tiny): the register-operand forward, four waves a
+  // 16-query tile (8.5 us a layer against 10.0 for the LDS-staged kernel; two waves 9.9, eight
+  // 9.5; the step 0.755 -> 0.751 ms). Its 16-byte loads need 16-byte aligned rows.
+  const auto al16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  if (!h16 && d == 64 && S == 128 && L % 16 == 0 && H % 4 == 0 && al16(q) && al16(k) && al16(v) && al16(mask) && al16(o)) {
+    dim3 grid(unsigned(B * heads), unsigned(L / 16));
+    MSX_LAUNCH(k_attn_fwd_reg<4>, grid, dim3(256), 0, s, q, k, v, mask, o, stats, int(L), int(H), int(heads), scale);
+    return;
+  }
+  const AttnPlan plan = attn_plan(B * heads, L, S, d, h16);
+  dim3 grid(unsigned(B * heads), row_blocks(L, plan));
 #define GO_H(T, W) launch_fwd_h<D, T, W>(s, grid, q, k, v, mask, o, stats, int(L), int(S), int(H), int(heads), scale)
 #define GO_F(T, W, KS) \
   launch_fwd<D, T, W, KS>(s, grid, plan.one, q, k, v, mask, o, stats, int(L), int(S), int(H), int(heads), scale)
 #define GO(D_) { constexpr int D = D_; MSX_BY_PLAN(plan, h16, GO_H, GO_F) }
-    MSX_BY_D(d, GO)
+  MSX_BY_D(d, GO)
 #undef GO
 #undef GO_F
 #undef GO_H
-    return;
-  }
-  if (scalar_fwd_lds(S, d) > kLdsMax || stats) refuse("attention shape outside the kernels' LDS budget");
-  dim3 grid(unsigned(B * heads), unsigned((L + 63) / 64));
-  size_t lds = scalar_fwd_lds(S, d);
-#define GO(D) MSX_LAUNCH(k_attn_fwd_scalar<D>, grid, dim3(64), lds, s, q, k, v, mask, o, int(L), int(S), int(H), int(heads), scale)
-  MSX_BY_D(d, GO)
-#undef GO
 }
 
 void attention_bwd(hipStream_t s, const float* q, const float* k, const float* v, const float* mask, const float* o,
@@ -1429,65 +1266,54 @@ void attention_bwd(hipStream_t s, const float* q, const float* k, const float* v
   int64_t d = H / heads;
   if (!head_ok(d) || L > S) refuse("attention head width or query rows");
   float scale = 1.0f / sqrtf(float(d));
-  if (attention_mfma(L, S, d)) {
-    if (!o || !stats || !dsum) refuse("the MFMA attention backward needs the forward output and statistics");
-    if (!dq) refuse("the MFMA attention backward computes d_i in its dQ pass: dQ is required");
-    const AttnPlan pq = attn_plan(B * heads, L, S, d, h16);
-    dim3 gq(unsigned(B * heads), row_blocks(L, pq));
-    if (!h16 && dk && dv && L == S) {
-      // Self-attention in f32: one launch for both passes (the key pass plans as the query pass).
-      dim3 gb(unsigned(B * heads), 2 * row_blocks(L, pq));
+  if (!bwd_fits(L, S, d)) refuse("attention shape outside the kernels' LDS budget");
+  h16 = h16 && whole_tiles(L, S);
+  if (!o || !stats || !dsum) refuse("the MFMA attention backward needs the forward output and statistics");
+  if (!dq) refuse("the MFMA attention backward computes d_i in its dQ pass: dQ is required");
+  const AttnPlan pq = attn_plan(B * heads, L, S, d, h16);
+  dim3 gq(unsigned(B * heads), row_blocks(L, pq));
+  if (!h16 && dk && dv && L == S) {
+    // Self-attention in f32: one launch for both passes (the key pass plans as the query pass).
+    dim3 gb(unsigned(B * heads), 2 * row_blocks(L, pq));
 #define GO_H(T, W)
 #define GO_F(T, W, KS)                                                                                              \
   launch_bwd<D, T, W, KS>(s, gb, row_blocks(L, pq), pq.one, q, k, v, mask, o, stats, g, dq, dk, dv, int(L), int(S), \
-                          int(H), int(heads), scale)
+                        int(H), int(heads), scale)
 #define GO(D_) { constexpr int D = D_; MSX_BY_PLAN(pq, false, GO_H, GO_F) }
-      MSX_BY_D(d, GO)
-#undef GO
-#undef GO_F
-#undef GO_H
-      return;
-    }
-#define GO_H(T, W) \
-  launch_bwd_q_h<D, T, W>(s, gq, q, k, v, mask, o, stats, g, dq, dsum, int(L), int(S), int(H), int(heads), scale)
-#define GO_F(T, W, KS)                                                                                            \
-  launch_bwd_q<D, T, W, KS>(s, gq, pq.one, q, k, v, mask, o, stats, g, dq, dsum, int(L), int(S), int(H), int(heads), \
-                            scale)
-#define GO(D_) { constexpr int D = D_; MSX_BY_PLAN(pq, h16, GO_H, GO_F) }
     MSX_BY_D(d, GO)
 #undef GO
 #undef GO_F
 #undef GO_H
-    if (dk || dv) {
-      const AttnPlan pk = attn_plan(B * heads, S, L, d, h16);
-      dim3 gk(unsigned(B * heads), row_blocks(S, pk));
+    return;
+  }
+#define GO_H(T, W) \
+  launch_bwd_q_h<D, T, W>(s, gq, q, k, v, mask, o, stats, g, dq, dsum, int(L), int(S), int(H), int(heads), scale)
+#define GO_F(T, W, KS)                                                                                            \
+  launch_bwd_q<D, T, W, KS>(s, gq, pq.one, q, k, v, mask, o, stats, g, dq, dsum, int(L), int(S), int(H), int(heads), \
+                          scale)
+#define GO(D_) { constexpr int D = D_; MSX_BY_PLAN(pq, h16, GO_H, GO_F) }
+  MSX_BY_D(d, GO)
+#undef GO
+#undef GO_F
+#undef GO_H
+  if (dk || dv) {
+    const AttnPlan pk = attn_plan(B * heads, S, L, d, h16);
+    dim3 gk(unsigned(B * heads), row_blocks(S, pk));
 #define GO_H(T, W) \
   launch_bwd_kv_h<D, T, W>(s, gk, q, k, v, mask, stats, g, dsum, dk, dv, int(L), int(S), int(H), int(heads), scale)
 #define GO_F(T, W, KS)                                                                                             \
   launch_bwd_kv<D, T, W, KS>(s, gk, pk.one, q, k, v, mask, stats, g, dsum, dk, dv, int(L), int(S), int(H), int(heads), \
-                             scale)
+                           scale)
 #define GO(D_) { constexpr int D = D_; MSX_BY_PLAN(pk, h16, GO_H, GO_F) }
-      MSX_BY_D(d, GO)
+    MSX_BY_D(d, GO)
 #undef GO
 #undef GO_F
 #undef GO_H
-    }
-    return;
   }
-  if (scalar_bwd_lds(L, S, d) > kLdsMax) refuse("attention shape outside the kernels' LDS budget");
-  size_t lds = scalar_bwd_lds(L, S, d);
-  int threads = int(std::min<int64_t>(256, std::max<int64_t>(64, (S + 63) / 64 * 64)));
-#define GO(D) MSX_LAUNCH(k_attn_bwd_scalar<D>, dim3(unsigned(B * heads)), dim3(threads), lds, s, q, k, v, mask, g, dq, dk, dv, int(L), int(S), int(H), int(heads), scale)
-  MSX_BY_D(d, GO)
-#undef GO
 }
 
 void prepare_attention() {
   const void* kernels[] = {
-      reinterpret_cast<const void*>(k_attn_fwd_scalar<16>), reinterpret_cast<const void*>(k_attn_fwd_scalar<32>),
-      reinterpret_cast<const void*>(k_attn_fwd_scalar<64>), reinterpret_cast<const void*>(k_attn_fwd_scalar<128>),
-      reinterpret_cast<const void*>(k_attn_bwd_scalar<16>), reinterpret_cast<const void*>(k_attn_bwd_scalar<32>),
-      reinterpret_cast<const void*>(k_attn_bwd_scalar<64>), reinterpret_cast<const void*>(k_attn_bwd_scalar<128>),
 #define MSX_ATTN_W(D, T, W)                                         \
   reinterpret_cast<const void*>(k_attn_fwd_mfma<D, T, W>),          \
       reinterpret_cast<const void*>(k_attn_bwd_q_mfma<D, T, W>),    \

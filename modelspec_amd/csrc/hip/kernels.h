@@ -220,7 +220,7 @@ void dropout(hipStream_t s, const float* x, float* o, int64_t n, const int32_t* 
 
 // Attention over a key mask [B, S]; q [B*L, H], k/v [B*S, H] (attention.hip).
 bool attention_fits(int64_t s, int64_t d);
-bool attention_mfma(int64_t L, int64_t S, int64_t d);  // the MFMA path runs (else the scalar one)
+
 // stats: [B*heads*L, 2] softmax maximum and sum per query (written when non-null; required by the
 // MFMA backward).
 // h16 (mixed precision): the MFMA path's contractions on the f16 MFMA with f32 accumulation.

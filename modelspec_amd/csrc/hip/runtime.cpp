@@ -1570,7 +1570,6 @@ void Executor::build() {
         if (!hk::attention_fits(S, H / heads)) throw IrError("attention shape has no HIP kernel (head width or sequence too large)");
         if (p.node(mask).op == Op::Input) key_masks_.push_back(p.node(mask).name);
         auto fkey = std::vector<uint32_t>{q, kv, v, mask, uint32_t(heads)};
-        bool mfma = hk::attention_mfma(L, S, H / heads);
         const bool h16 = s_.opt_.mixed;  // mixed precision: the f16 MFMA
         if (flash(x)) {
           // The f16 attention on the operands' f16 copies, writing its outputs' copies itself.
@@ -1632,11 +1631,10 @@ void Executor::build() {
           break;
         }
         if (x.op == Op::Attention) {
-          void* st2 = mfma ? R(size_t(B * heads * L) * 8) : nullptr;
+          void* st2 = R(size_t(B * heads * L) * 8);
           attn_fwd[fkey] = {id, st2};
           push([=](hipStream_t s) {
-            hk::attention_fwd(s, F(q), F(kv), F(v), F(mask), F(id), st2 ? static_cast<float*>(A(st2)) : nullptr, B, L, S, H, heads,
-                              h16);
+            hk::attention_fwd(s, F(q), F(kv), F(v), F(mask), F(id), static_cast<float*>(A(st2)), B, L, S, H, heads, h16);
           });
           pending.back().pure = true;
           break;
@@ -1654,29 +1652,26 @@ void Executor::build() {
         // Attention over the same operands, else a forward run into scratch first.
         int64_t fwd_out = -1;
         void *stats_tok = nullptr, *scratch_o = nullptr, *dsum = nullptr, *dq_scratch = nullptr;
-        if (mfma) {
-          auto f = attn_fwd.find(fkey);
-          if (f != attn_fwd.end()) {
-            fwd_out = int64_t(f->second.first);
-            stats_tok = f->second.second;
-          } else {
-            scratch_o = R(size_t(shape(q)[0] * H) * 4);
-            stats_tok = R(size_t(B * heads * L) * 8);
-            push([=](hipStream_t s) {
-              hk::attention_fwd(s, F(q), F(kv), F(v), F(mask), static_cast<float*>(A(scratch_o)),
-                                static_cast<float*>(A(stats_tok)), B, L, S, H, heads, h16);
-            });
-          }
-          dsum = R(size_t(B * heads * L) * 4);
-          if (members[0] < 0) dq_scratch = R(size_t(shape(q)[0] * H) * 4);
+        auto f = attn_fwd.find(fkey);
+        if (f != attn_fwd.end()) {
+          fwd_out = int64_t(f->second.first);
+          stats_tok = f->second.second;
+        } else {
+          scratch_o = R(size_t(shape(q)[0] * H) * 4);
+          stats_tok = R(size_t(B * heads * L) * 8);
+          push([=](hipStream_t s) {
+            hk::attention_fwd(s, F(q), F(kv), F(v), F(mask), static_cast<float*>(A(scratch_o)),
+                              static_cast<float*>(A(stats_tok)), B, L, S, H, heads, h16);
+          });
         }
+        dsum = R(size_t(B * heads * L) * 4);
+        if (members[0] < 0) dq_scratch = R(size_t(shape(q)[0] * H) * 4);
         push([=](hipStream_t s) {
           auto out = [&](int64_t v2) { return v2 >= 0 ? F(uint32_t(v2)) : nullptr; };
-          float* dq = members[0] >= 0 ? F(uint32_t(members[0])) : (dq_scratch ? static_cast<float*>(A(dq_scratch)) : nullptr);
-          const float* fo = fwd_out >= 0 ? F(uint32_t(fwd_out)) : (scratch_o ? static_cast<float*>(A(scratch_o)) : nullptr);
-          hk::attention_bwd(s, F(q), F(kv), F(v), F(mask), fo, stats_tok ? static_cast<float*>(A(stats_tok)) : nullptr, F(g), dq,
-                            out(members[1]), out(members[2]), dsum ? static_cast<float*>(A(dsum)) : nullptr, B, L, S, H, heads,
-                            h16);
+          float* dq = members[0] >= 0 ? F(uint32_t(members[0])) : static_cast<float*>(A(dq_scratch));
+          const float* fo = fwd_out >= 0 ? F(uint32_t(fwd_out)) : static_cast<float*>(A(scratch_o));
+          hk::attention_bwd(s, F(q), F(kv), F(v), F(mask), fo, static_cast<float*>(A(stats_tok)), F(g), dq, out(members[1]),
+                            out(members[2]), static_cast<float*>(A(dsum)), B, L, S, H, heads, h16);
         });
         pending.back().pure = true;
         break;
