@@ -28,6 +28,7 @@ SOURCES = [
     "hip/kernels.hip",
     "hip/gemm.hip",
     "hip/gemm_lds.hip",
+    "hip/gemm16.hip",
     "hip/attention.hip",
     "hip/flash16.hip",
     "hip/data.hip",
@@ -45,6 +46,7 @@ FLAGS = [
 # Per-source flags. The direct-to-LDS GEMMs and the f16 attention keep their MFMA accumulators in VGPRs: with the
 # compiler's default choice (AGPRs) it rotated the accumulators through copies every K tile.
 FILE_FLAGS = {"hip/gemm_lds.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+              "hip/gemm16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
               "hip/flash16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 

@@ -438,37 +438,36 @@ namespace {
 // The tile shape and split-K of a GEMM, from measured MI355X timings of the step's shapes: large
 // outputs (and very deep K) take 64 x 64 tiles, outputs up to 2^19 elements 32 x 32, the rest
 // 32 x 64. Split-K, whose slice sum costs a launch unless deferred to a batched finalize, is used
-// when deferred or when K is deep, to fill the chip. The f16 MFMA does eight times the work of
-// the f32 one an instruction, so mixed-precision GEMMs of 2^21 outputs or more (or K of 8192 or
-// more) take 128 x 128 tiles: four times the MFMAs per operand byte staged.
+// when deferred or when K is deep, to fill the chip.
 struct SplitPlan { int wm, wn, wk, split; int64_t chunk; };
 SplitPlan split_plan(int64_t m, int64_t n, int64_t k, bool defer, bool h16, bool ce = false) {
   const int64_t mn = m * n;
   SplitPlan p{};
-  // A cross-entropy head (ce) always takes the largest tile, the one its kernels are built for.
-  // Mixed precision: the 128 x 128 tiles of k_gemm_lds16 (and k_gemm_w's largest f16 tile).
+  // Mixed precision: k_gemm_w's largest f16 tile (where gemm16 does not take the problem).
   if (h16) { p.wm = 4; p.wn = 4; p.wk = 32; }
+  // A cross-entropy head (ce) always takes the largest tile, the one its kernels are built for.
   else if (ce || mn >= (int64_t(1) << 21) || k >= 8192) { p.wm = 2; p.wn = 2; p.wk = 16; }
   else if (mn <= (int64_t(1) << 19)) { p.wm = 1; p.wn = 1; p.wk = 32; }
   else { p.wm = 1; p.wn = 2; p.wk = 16; }
+  if (h16 && !ce) {
+    const Split16 q = gemm16_split(m, n, k, defer);
+    p.split = q.split;
+    p.chunk = q.chunk;
+    return p;
+  }
   const int64_t tiles = ((m + 32 * p.wm - 1) / (32 * p.wm)) * ((n + 32 * p.wn - 1) / (32 * p.wn));
   int64_t want = 1;
   if (defer || k >= 1024) {
-    const int64_t blocks = p.wm == 2 ? 2048 : 1024;  // 128 x 128 tiles: 1024 (4 a CU)
+    const int64_t blocks = p.wm == 2 ? 2048 : 1024;
     want = tiles < blocks / 4 ? (blocks + tiles - 1) / tiles : 1;
     // An f32 product of K 8192 or more summed by its own launch (BERT-tiny's decoder input
     // gradient, K 30522): half as many slices, 74 -> 37 (A/B in one run: 74 -> 68 us, half the
     // partials written and read back; a quarter as many 74 us, 1.5 times as many 81 us).
-    if (!h16 && !defer && k >= 8192) want = std::max<int64_t>(1, want / 2);
+    if (!defer && k >= 8192) want = std::max<int64_t>(1, want / 2);
   }
-  // Deferred slices keep 128 K steps or more (4096 for 128 x 128 tiles, whose f16 blocks get
-  // through K fastest): their partials all go through the finalize, m n floats a slice
-  // (BERT-base's K = 16384 weight gradients: 4 slices 37.7 ms a step, 16 slices 38.0, 2 slices
-  // 38.1).
-  // (A deferred f16 product of K under 8192 takes slices of at least 512: BERT-base's head dense
-  // weight gradient, 768x768 at K = 2880, otherwise runs 36 blocks.)
-  const int64_t min_slice = defer ? (p.wm == 4 ? (k >= 8192 ? 4096 : 512) : 128) : 64;
-  const int64_t split = std::max<int64_t>(1, std::min(want, k / min_slice));
+  // Deferred slices keep 128 K steps or more: their partials all go through the finalize, m n
+  // floats a slice.
+  const int64_t split = std::max<int64_t>(1, std::min(want, k / (defer ? 128 : 64)));
   p.chunk = ((k + split - 1) / split + kSliceAlign - 1) / kSliceAlign * kSliceAlign;
   p.split = int((k + p.chunk - 1) / p.chunk);
   return p;
@@ -501,9 +500,8 @@ int gemm_deferred_jobs(const GemmArgs& g, ColumnJob* jobs) {
   return 2;
 }
 
-bool gemm_lds16_fits(const GemmArgs& g) {
-  if (!g.h16 || g.ksegs > 1 || g.ce_operand || g.ce_part || g.m <= 0 || g.n <= 0 || g.k <= 0) return false;
-  return lds16_layout(g, split_plan(g.m, g.n, g.k, g.defer, true, false).chunk);
+bool gemm16_fits(const GemmArgs& g) {
+  return g.h16 && !g.ce_operand && !g.ce_part && g.m > 0 && g.n > 0 && g.k > 0 && gemm16_layout(g);
 }
 
 void gemm(hipStream_t s, const GemmArgs& g) { gemm_group(s, &g, 1); }
@@ -570,6 +568,8 @@ void gemm_group(hipStream_t s, const GemmArgs* list, int count) {
     for (int q = 0; q < ksegs; ++q) {
       ptrs.a[q] = g.seg_a[q];
       ptrs.b[q] = g.seg_b[q];
+      ptrs.a16[q] = g.seg_a16[q];
+      ptrs.b16[q] = g.seg_b16[q];
     }
   float* ws = ptrs.ws[0];
   // Tiles in the grouped order: split slices outermost; within a slice the tiles that share the
@@ -659,14 +659,14 @@ void gemm_group(hipStream_t s, const GemmArgs* list, int count) {
   else if (plan.wn == 2) MSX_KS_V(TA, TB, 1, 2, 16);        \
   else MSX_KS_V(TA, TB, 1, 1, 32);
   // The large f32 shapes take k_gemm_lds when their layout allows it, mixed-precision GEMMs whose
-  // operands both have f16 copies k_gemm_lds16 (gemm_lds.hip).
+  // operands both have f16 copies the kernels of gemm16.hip.
   bool f16_out = false;  // the launched kernel writes the f16 output copies itself
   const bool lds = !g.h16 && ksegs == 1 && count == 1 && !ce && gemm_lds(s, g, ptrs, split, chunk);
-  const bool lds16 = !lds && g.h16 && ksegs == 1 && !ce && gemm_lds16(s, list, count, ptrs, split, chunk);
+  const bool lds16 = !lds && g.h16 && !ce && gemm16(s, list, count, ptrs, split, chunk);
   if (lds16) f16_out = true;
   for (int q = 0; q < count && !lds16; ++q)
-    if (!list[q].a || !list[q].b || !list[q].c)
-      bad("a GEMM on an f16-only operand or output needs k_gemm_lds16 (f16 copies, its layout)");
+    if ((ksegs == 1 && (!list[q].a || !list[q].b)) || !list[q].c)
+      bad("a GEMM on an f16-only operand or output needs gemm16 (f16 copies, its layout)");
   if (lds || lds16) {
     // launched
   } else if (ksegs > 1) {
@@ -681,7 +681,7 @@ void gemm_group(hipStream_t s, const GemmArgs* list, int count) {
     if (g.h16) { MSX_CE(4, 4, 32, true) }
     else { MSX_CE(2, 2, 16, false) }
   } else if (g.h16) {
-    if (g.colsum) bad("mixed-precision column sums need k_gemm_lds16's layout (f16 copies, K a multiple of 32)");
+    if (g.colsum) bad("mixed-precision column sums need gemm16's layout (f16 copies, rows of whole 16-byte groups)");
     if (!g.ta && !g.tb) { MSX_WIDE_HT(false, false) }
     else if (g.ta && !g.tb) { MSX_WIDE_HT(true, false) }
     else if (!g.ta && g.tb) { MSX_WIDE_HT(false, true) }

@@ -1,4 +1,4 @@
-// Device pieces shared by the two GEMM sources (gemm.hip, gemm_lds.hip): the output epilogue and
+// Device pieces shared by the GEMM sources (gemm.hip, gemm_lds.hip, gemm16.hip): the output epilogue and
 // the tile order, and the large-shape kernel's launcher.
 #pragma once
 #include "kernels.h"
@@ -97,12 +97,18 @@ struct GemmOrder {
 // with the caller's split-K slices (`split` slices of `chunk` K, partials in ptrs.ws[0]) when its
 // shape and layout suit it; returns false, launching nothing, otherwise.
 bool gemm_lds(hipStream_t s, const GemmArgs& g, const GemmPtrs& ptrs, int split, int64_t chunk);
-// The same for a mixed-precision group whose operands all have f16 copies (GemmArgs::a16, b16):
-// the f16 kernel reads them straight into LDS; it writes the f32 output (or split-K partials) and
-// the f16 output copies asked for.
-bool gemm_lds16(hipStream_t s, const GemmArgs* list, int count, const GemmPtrs& ptrs, int split, int64_t chunk);
-// Whether k_gemm_lds16 takes a problem of this shape and layout with split-K slices of `chunk`
-// (its f16 operand copies present and 16-byte aligned aside).
-bool lds16_layout(const GemmArgs& g, int64_t chunk);
+// The same for a mixed-precision group (or the K segments of one problem) whose operands all have f16
+// copies (GemmArgs::a16, b16; gemm16.hip): it writes the f32 output (or split-K partials) and the
+// f16 output copies asked for.
+bool gemm16(hipStream_t s, const GemmArgs* list, int count, const GemmPtrs& ptrs, int split, int64_t chunk);
+// Whether gemm16 takes a problem of this layout (its f16 operand copies present and 16-byte aligned
+// aside): rows of whole 16-byte groups.
+bool gemm16_layout(const GemmArgs& g);
+// The split-K slices of a mixed-precision product.
+struct Split16 {
+  int split;
+  int64_t chunk;
+};
+Split16 gemm16_split(int64_t m, int64_t n, int64_t k, bool defer);
 
 }  // namespace msx::hk

@@ -319,309 +319,6 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_lds(GemmPtrs ptrs, int6
 }
 
 // ---------------------------------------------------------------------------------------------
-// The mixed-precision GEMM on f16 operands in HBM (k_gemm_lds16): K tiles of 32 halves move straight
-// into a 3-stage LDS ring as in k_gemm_lds, and v_mfma_f32_16x16x32_f16 takes 8 consecutive K of a
-// row a lane, f32 accumulation.
-//   - An operand contiguous along K (KC) is staged [row][32 K]: 64 bytes a row, its 16-byte chunk
-//     kq at slot kq ^ ((row >> 2) & 3), so the 16 rows a quarter-wave reads at one chunk hit
-//     distinct banks; lane (c, q) reads row c's chunk q with one 16-byte read.
-//   - An operand contiguous along its rows is staged [K][rows] as in memory, the 16-byte chunk ch of
-//     K row k at ch ^ 2 (k mod 4) within its group of 8 (128 bytes). A lane's 8 K of one row come
-//     from two ds_read_b64_tr_b16: in each 16-lane group, source lane l reads 4 rows x 1 K (8 bytes)
-//     at K row k0 + l / 4, rows base + 4 (l mod 4) .. + 3, and after the transpose lane c holds row
-//     base + c at K k0 .. k0 + 3.
-// Lane (c, q) thus supplies row c of its 16-row block at K 8q .. 8q + 7 in both layouts, and holds
-// output rows 16 i + c, columns 16 j + 4 q .. + 3 (the MFMA takes B's fragment first: C^T tiles).
-// K must be a multiple of 32, or the K-contiguous operands zero-padded to it; the K rows of an
-// operand along its rows are clamped to the last (their products with the padding vanish).
-
-template <int BM, int BN, int WGM, int WGN, bool AKC, bool BKC, int NS, int SUMS, int MF = 16, int BK = 32>
-__global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_lds16(GemmPtrs ptrs, int64_t M, int64_t N, int64_t K,
-                                                               int64_t lda, int64_t ldb, int64_t ldc, int64_t kchunk,
-                                                               int64_t zero_to, bool vo, GemmOrder order) {
-  constexpr int W = WGM * WGN;
-  static_assert(BK == 32 || BK == 64, "K tiles of 32 or 64 halves");
-  constexpr int WTM = BM / WGM, WTN = BN / WGN, I = WTM / MF, J = WTN / MF;
-  static_assert(MF == 16 || MF == 32, "16x16x32 or 32x32x16 MFMA blocks");
-  static_assert(I >= 1 && J >= 1 && WTM % MF == 0 && WTN % MF == 0, "whole MFMA blocks a wave");
-  // MFMA blocks of MF rows: 16x16x32 (KS = 1 K step of 32 a tile) or 32x32x16 (KS = 2 of 16).
-  constexpr int KS = BK / (MF == 16 ? 32 : 16), NV = MF == 16 ? 4 : 16;
-  // A K-contiguous tile's rows: CPR 16-byte chunks (BK 32: 64 bytes, BK 64: a whole 128-byte line),
-  // RPI rows a 1 KB load instruction; chunk c of row r at slot c ^ swz(r).
-  constexpr int CPR = BK / 8, RPI = 64 / CPR;
-  typedef float vacc __attribute__((ext_vector_type(NV)));
-  constexpr int SA = BM * BK, SB = BN * BK, SS = SA + SB;  // halves a stage
-  constexpr int LA = SA / 512, LB = SB / 512;               // 1 KB wave load instructions a tile
-  static_assert(LA % W == 0 && LB % W == 0, "whole load instructions a wave");
-  constexpr int PA = LA / W, PB = LB / W, LPT = PA + PB;
-  __shared__ __align__(16) _Float16 smem[NS * SS];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, q = lane >> 4;
-  const uint32_t per = gridDim.x / 8, tg = (blockIdx.x % 8) * per + blockIdx.x / 8;
-  if (tg >= order.tiles * uint32_t(ptrs.count)) return;
-  // The problem of the group, then its tile.
-  const int qp = int(tg / order.tiles);
-  const uint32_t t0 = tg - uint32_t(qp) * order.tiles;
-  const uint32_t tz = t0 / (order.mt * order.nt), tr = t0 % (order.mt * order.nt);
-  const uint32_t tm = order.m_fastest ? tr % order.mt : tr / order.nt;
-  const uint32_t tn = order.m_fastest ? tr / order.mt : tr % order.nt;
-  const int64_t m0 = int64_t(tm) * BM, n0 = int64_t(tn) * BN;
-  const int64_t kpad = (K + BK - 1) / BK * BK;
-  const int64_t kbeg = int64_t(tz) * kchunk, kend = kpad < kbeg + kchunk ? kpad : kbeg + kchunk;
-  const int tiles = int((kend - kbeg) / BK);
-  const int wm = (wave / WGN) * WTM, wn = (wave % WGN) * WTN;
-  const _Float16* __restrict__ A = ptrs.a16[qp];
-  const _Float16* __restrict__ B = ptrs.b16[qp];
-  const GemmEpi epi = ptrs.epi[qp];
-  float* __restrict__ ws = ptrs.ws[qp];
-  float* __restrict__ colsum = ptrs.colsum[qp];
-  auto swz = [](int r) { return BK == 32 ? ((r >> 2) & 3) : (r & 7); };
-  const int64_t kmax = K - 1;
-  const _Float16* srcA[PA];
-  const _Float16* srcB[PB];
-  int kofA[PA], kofB[PB];
-#pragma unroll
-  for (int h = 0; h < PA; ++h) {
-    const int t = wave * PA + h;
-    if (AKC) {
-      const int r = t * RPI + lane / CPR, ch = (lane % CPR) ^ swz(r);
-      const int64_t row = m0 + r < M ? m0 + r : M - 1;
-      srcA[h] = A + row * lda + kbeg + 8 * ch;
-      kofA[h] = 0;
-    } else {
-      constexpr int RQ = BM / 8, KR = 512 / BM;
-      const int kr = t * KR + lane / RQ, slot = lane % RQ;
-      const int ch = (slot & ~7) | ((slot & 7) ^ (2 * (kr & 3)));
-      int64_t col = m0 + 8 * ch;
-      col = col < M ? col : ((M - 1) & ~int64_t(7));
-      srcA[h] = A + col;
-      kofA[h] = kr;
-    }
-  }
-#pragma unroll
-  for (int h = 0; h < PB; ++h) {
-    const int t = wave * PB + h;
-    if (BKC) {
-      const int r = t * RPI + lane / CPR, ch = (lane % CPR) ^ swz(r);
-      const int64_t row = n0 + r < N ? n0 + r : N - 1;
-      srcB[h] = B + row * ldb + kbeg + 8 * ch;
-      kofB[h] = 0;
-    } else {
-      constexpr int RQ = BN / 8, KR = 512 / BN;
-      const int kr = t * KR + lane / RQ, slot = lane % RQ;
-      const int ch = (slot & ~7) | ((slot & 7) ^ (2 * (kr & 3)));
-      int64_t col = n0 + 8 * ch;
-      col = col < N ? col : ((N - 1) & ~int64_t(7));
-      srcB[h] = B + col;
-      kofB[h] = kr;
-    }
-  }
-  auto issue = [&](int tile) {
-    tile = tile < tiles ? tile : tiles - 1;
-    _Float16* st = smem + (tile % NS) * SS;
-    const int64_t k0 = int64_t(tile) * BK;
-#pragma unroll
-    for (int h = 0; h < PA; ++h) {
-      const int t = wave * PA + h;
-      const int64_t kr = kbeg + k0 + kofA[h];
-      const _Float16* src = AKC ? srcA[h] + k0 : srcA[h] + (kr < kmax ? kr : kmax) * lda;
-      load_lds16(reinterpret_cast<const float*>(src), reinterpret_cast<float*>(st + t * 512));
-    }
-#pragma unroll
-    for (int h = 0; h < PB; ++h) {
-      const int t = wave * PB + h;
-      const int64_t kr = kbeg + k0 + kofB[h];
-      const _Float16* src = BKC ? srcB[h] + k0 : srcB[h] + (kr < kmax ? kr : kmax) * ldb;
-      load_lds16(reinterpret_cast<const float*>(src), reinterpret_cast<float*>(st + SA + t * 512));
-    }
-  };
-  vacc acc[I][J];
-#pragma unroll
-  for (int i = 0; i < I; ++i)
-#pragma unroll
-    for (int j = 0; j < J; ++j)
-#pragma unroll
-      for (int e = 0; e < NV; ++e) acc[i][j][e] = 0.0f;
-  // Lane roles. MF 16: lane (c = l mod 16, q = l / 16) supplies row c of a 16-row block at K
-  // 8 q .. 8 q + 7. MF 32: lane (c = l mod 32, h = l / 32) supplies row c of a 32-row block at K
-  // 16 ks + 8 h .. + 7 of K step ks. Either way the lane's 8 K are one 16-byte chunk kq (kq = q,
-  // or 2 ks + h) of the row.
-  const int fc = MF == 16 ? c : lane & 31, fh = MF == 16 ? q : lane >> 5;
-  auto kc_frag = [&](const _Float16* S, int r, int kq) {
-    return *reinterpret_cast<const v8h*>(S + r * BK + 8 * (kq ^ swz(r)));
-  };
-  // The LDS address of the transposed read of K rows k0 .. k0 + 3 of the 16 rows from base: in each
-  // 16-lane group, source lane li reads K row k0 + li / 4, rows base + 4 (li mod 4) .. + 3.
-  auto tr_at = [&](const _Float16* S, int R, int base, int k0) {
-    const int k = k0 + c / 4;
-    const int row = base + 4 * (c % 4);
-    const int ch = row / 8, slot = (ch & ~7) | ((ch & 7) ^ (2 * (k & 3)));
-    return lds_at(S + k * R + slot * 8 + (row % 8));
-  };
-  // The transposed reads (base row, first K row) of one 8-half fragment of this lane: MF 16, rows
-  // base .. + 15 at K 8 q + {0, 4}; MF 32, rows base + 16 (g mod 2) .. (g = l / 16) at K
-  // 16 ks + 8 (g / 2) + {0, 4}.
-  auto tr_pair = [&](int base, int ks, int hh, int& rb, int& k0) {
-    if constexpr (MF == 16) {
-      rb = base;
-      k0 = 32 * ks + 8 * q + 4 * hh;
-    } else {
-      rb = base + 16 * (q & 1);
-      k0 = 16 * ks + 8 * (q >> 1) + 4 * hh;
-    }
-  };
-  static_assert((AKC || (I * KS) % 4 == 0) && (BKC || (J * KS) % 4 == 0),
-                "an operand along its rows takes its fragments in fours");
-  // Fragments (ks, u) of an operand along its rows, rows base0 + MF u, eight transposed reads a group
-  // of four.
-  auto tr_frags = [&](const _Float16* S, int R, int base0, auto& out) {
-    constexpr int U = sizeof(out[0]) / sizeof(out[0][0]);
-    constexpr int G = KS * U / 4;
-#pragma unroll
-    for (int g4 = 0; g4 < G; ++g4) {
-      uint32_t at[8];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int fi = 4 * g4 + e, ks = fi / U, u = fi % U;
-#pragma unroll
-        for (int hh = 0; hh < 2; ++hh) {
-          int rb, k0;
-          tr_pair(base0 + MF * u, ks, hh, rb, k0);
-          at[2 * e + hh] = tr_at(S, R, rb, k0);
-        }
-      }
-      v4s16 r[8];
-      tr_read16x8(at, r);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int fi = 4 * g4 + e, ks = fi / U, u = fi % U;
-        const v4h16 lo = __builtin_bit_cast(v4h16, r[2 * e]), hi = __builtin_bit_cast(v4h16, r[2 * e + 1]);
-        out[ks][u] = v8h{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      }
-    }
-  };
-  struct Frag { v8h a[KS][I], b[KS][J]; };
-  auto read = [&](int tile, Frag& f) {
-    const _Float16* As = smem + (tile % NS) * SS;
-    const _Float16* Bs = As + SA;
-    if constexpr (AKC) {
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-        for (int i = 0; i < I; ++i) f.a[ks][i] = kc_frag(As, wm + MF * i + fc, MF == 16 ? 4 * ks + q : 2 * ks + fh);
-    } else {
-      tr_frags(As, BM, wm, f.a);
-    }
-    if constexpr (BKC) {
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-        for (int j = 0; j < J; ++j) f.b[ks][j] = kc_frag(Bs, wn + MF * j + fc, MF == 16 ? 4 * ks + q : 2 * ks + fh);
-    } else {
-      tr_frags(Bs, BN, wn, f.b);
-    }
-  };
-  // Sums over K of this lane's operand rows (SUMS 1: op(A)'s rows, 2: op(B)'s columns, i.e. the
-  // fragments' rows), by the waves of the first wave column (row), which read every row of the
-  // operand: the lane adds its 8 K of rows MF u + fc of the wave tile, in K order.
-  constexpr int SN = SUMS == 1 ? I : SUMS == 2 ? J : 1;
-  float ksum[SN];
-#pragma unroll
-  for (int u = 0; u < SN; ++u) ksum[u] = 0.0f;
-  const bool sum_wave = SUMS == 1 ? wn == 0 : SUMS == 2 ? wm == 0 : false;
-#pragma unroll
-  for (int p = 0; p < NS - 1; ++p) issue(p);
-#pragma unroll 1
-  for (int t = 0; t < tiles; ++t) {
-    wait_vm((NS - 2) * LPT);
-    __builtin_amdgcn_s_barrier();
-    issue(t + NS - 1);
-    Frag f;
-    read(t, f);
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-      for (int i = 0; i < I; ++i)
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-          if constexpr (MF == 16)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.b[ks][j], f.a[ks][i], acc[i][j], 0, 0, 0);
-          else
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.b[ks][j], f.a[ks][i], acc[i][j], 0, 0, 0);
-        }
-    if (SUMS != 0 && sum_wave) {
-#pragma unroll
-      for (int u = 0; u < SN; ++u) {
-        // v_dot2_f32_f16 against (1, 1): two halves added into the f32 sum a VALU op.
-        typedef _Float16 v2h_ __attribute__((ext_vector_type(2)));
-        const v2h_ one{_Float16(1.0f), _Float16(1.0f)};
-        float x = ksum[u];
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          const v8h h = SUMS == 1 ? f.a[ks][u] : f.b[ks][u];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) x = __builtin_amdgcn_fdot2(v2h_{h[2 * e], h[2 * e + 1]}, one, x, false);
-        }
-        ksum[u] = x;
-      }
-    }
-  }
-  wait_vm(0);  // no load may still write LDS when the block ends
-  float* out = ws ? ws + int64_t(tz) * M * N : ptrs.c[qp];
-  _Float16* out16 = ws ? nullptr : ptrs.c16[qp];
-  const int64_t ldo = ws ? N : ldc, zto = ws ? N : zero_to;
-  const bool more = !ws && (epi.bias || epi.act != EPI_NONE || epi.addend || epi.drop_token);
-  // Output element (row, col) of block (i, j): the MFMA took B's fragment first, so the lane holds
-  // output row MF i + fc and, for each group g of 4 accumulators, the columns MF j + 8 g + 4 fh
-  // (MF 32) or 16 j + 4 q (MF 16) .. + 3.
-#pragma unroll
-  for (int i = 0; i < I; ++i) {
-    const int64_t row = m0 + wm + MF * i + fc;
-    if (row >= M) continue;
-#pragma unroll
-    for (int j = 0; j < J; ++j)
-#pragma unroll
-      for (int g = 0; g < NV / 4; ++g) {
-        const int64_t col = n0 + wn + MF * j + (MF == 16 ? 4 * q : 8 * g + 4 * fh);
-        float4 v = make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
-        if (vo && col + 3 < N) {
-          if (more) v = gemm_epilogue4(epi, v, row, col, ldo);
-          if (out) *reinterpret_cast<float4*>(out + row * ldo + col) = v;
-          if (out16)
-            *reinterpret_cast<v4h16*>(out16 + row * ldo + col) =
-                v4h16{_Float16(v.x), _Float16(v.y), _Float16(v.z), _Float16(v.w)};
-        } else {
-          const float vs[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            if (col + u >= zto) continue;
-            const float x = col + u < N ? (more ? gemm_epilogue(epi, vs[u], row, col + u, ldo) : vs[u]) : 0.0f;
-            if (out) out[row * ldo + col + u] = x;
-            if (out16) out16[row * ldo + col + u] = _Float16(x);
-          }
-        }
-      }
-  }
-  if constexpr (SUMS != 0) {
-    // The lane groups (q for MF 16, h for MF 32) hold disjoint K: added across them (fixed order),
-    // written by group 0 at row (column) base + MF u + fc; split-K slices into the workspace's
-    // sums, slice tz.
-#pragma unroll
-    for (int u = 0; u < SN; ++u) {
-      if constexpr (MF == 16) ksum[u] += __shfl_xor(ksum[u], 16, 64);
-      ksum[u] += __shfl_xor(ksum[u], 32, 64);
-    }
-    if (sum_wave && fh == 0 && colsum) {
-      const int64_t base = SUMS == 1 ? m0 + wm : n0 + wn, width = SUMS == 1 ? M : N;
-      float* dst = colsum + (ws ? int64_t(tz) * width : 0);
-#pragma unroll
-      for (int u = 0; u < SN; ++u) {
-        const int64_t at = base + MF * u + fc;
-        if (at < width) dst[at] = ksum[u];
-      }
-    }
-  }
-}
-
 namespace {
 // Whether k_gemm_lds can read this problem with K tiles of bk: 16-byte aligned operands and rows;
 // a K tail only where every operand contiguous along K (KC) is zero-padded to the next multiple of
@@ -689,65 +386,6 @@ bool gemm_lds(hipStream_t s, const GemmArgs& g, const GemmPtrs& ptrs, int split,
     return true;
   }
   return false;
-}
-
-bool lds16_layout(const GemmArgs& o, int64_t chunk) {
-  constexpr int BK = 32;
-  const bool akc = !o.ta, bkc = o.tb;
-  const int64_t kpad = (o.k + BK - 1) / BK * BK;
-  if (chunk % BK != 0 || o.lda % 8 != 0 || o.ldb % 8 != 0) return false;
-  // A K tail only over zero padding of the K-contiguous operands (the other kind is clamped, and
-  // a summed operand's clamped rows would enter its sums).
-  if (o.k % BK != 0 && ((!akc && !bkc) || (akc && !(o.pad_a && o.lda >= kpad)) || (bkc && !(o.pad_b && o.ldb >= kpad)) ||
-                        (o.colsum && !(o.sum_a ? akc : bkc))))
-    return false;
-  // An operand along its rows: whole 8-row chunks, or a pitch that holds the last one.
-  if (!akc && o.m % 8 != 0 && o.lda < (o.m + 7) / 8 * 8) return false;
-  if (!bkc && o.n % 8 != 0 && o.ldb < (o.n + 7) / 8 * 8) return false;
-  return true;
-}
-
-bool gemm_lds16(hipStream_t s, const GemmArgs* list, int count, const GemmPtrs& ptrs, int split, int64_t chunk) {
-  const GemmArgs& g = list[0];
-  auto a16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  const bool akc = !g.ta, bkc = g.tb;
-  for (int q = 0; q < count; ++q) {
-    const GemmArgs& o = list[q];
-    if (!o.a16 || !o.b16 || !a16(o.a16) || !a16(o.b16) || !lds16_layout(o, chunk)) return false;
-  }
-  constexpr int BM = 128, BN = 128;
-  const int64_t lmt = (g.m + BM - 1) / BM, lnt = (g.n + BN - 1) / BN;
-  const int64_t ltiles = lmt * lnt * split;
-  if (ltiles * count > (int64_t(1) << 30)) bad("gemm has too many tiles");
-  const GemmOrder lorder{uint32_t(lmt), uint32_t(lnt), uint32_t(ltiles), g.n * g.k >= g.m * g.k};
-  const dim3 lgrid(unsigned((ltiles * count + 7) / 8 * 8));
-  bool vo = true;
-  for (int q = 0; q < count; ++q) {
-    const GemmArgs& o = list[q];
-    vo = vo && (ptrs.ws[q] ? (o.n % 4 == 0 && a16(ptrs.ws[q]))
-                           : (o.ldc % 4 == 0 && a16(o.c) && a16(o.c16) && a16(o.bias) && a16(o.addend) && a16(o.pre_in) &&
-                              a16(o.pre_out) && a16(o.pre16)));
-  }
-  const int64_t zero_to = g.pad_c ? g.ldc : g.n;
-  const int sums = g.colsum ? (g.sum_a ? 1 : 2) : 0;
-  // 128x128 tiles, 2x2 waves, K tiles of 32 in a 2-stage ring, 16x16x32 blocks. Measured on the
-  // BERT-base step, A/B in one run on one box: a 3-stage ring 23.43 ms (2 stages 23.18); 32x32x16
-  // blocks 25.45; 4 stages 26.30; 256x128, 128x256 and 256x256 tiles 26.0, 25.8 and 26.6; K tiles
-  // of 64 (whole 128-byte rows of a K-contiguous operand a load) 24.6.
-#define MSX_L16S(AK, BKC_, S)                                                                                         \
-  MSX_LAUNCH((k_gemm_lds16<BM, BN, 2, 2, AK, BKC_, 2, S, 16, 32>), lgrid, dim3(256), 0, s, ptrs, g.m, g.n, g.k, g.lda, \
-             g.ldb, g.ldc, chunk, zero_to, vo, lorder);
-#define MSX_L16(AK, BKC_)                  \
-  if (sums == 1) { MSX_L16S(AK, BKC_, 1) }      \
-  else if (sums == 2) { MSX_L16S(AK, BKC_, 2) } \
-  else { MSX_L16S(AK, BKC_, 0) }
-  if (akc && bkc) { MSX_L16(true, true); }
-  else if (akc) { MSX_L16(true, false); }
-  else if (bkc) { MSX_L16(false, true); }
-  else { MSX_L16(false, false); }
-#undef MSX_L16
-#undef MSX_L16S
-  return true;
 }
 
 }  // namespace msx::hk

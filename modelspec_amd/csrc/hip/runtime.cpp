@@ -252,7 +252,7 @@ void Executor::build() {
   for (auto [m, t] : mm_transposed) transposed_out.insert(t);
   // A SumRows of a MatMul's un-transposed B operand (the bias gradient beside its weight gradient)
   // is taken by that GEMM from its LDS tiles, when no reader of the sum comes before the GEMM.
-  // Under mixed precision only the f16 GEMM on the operands' f16 copies (k_gemm_lds16) takes the
+  // Under mixed precision only the f16 GEMM on the operands' f16 copies (gemm16) takes the
   // sums (of the f16 values): both operands' rows whole 16-byte groups of f16, K a multiple of 32.
   std::map<uint32_t, uint32_t> colsum_of;  // MatMul -> SumRows
   std::set<uint32_t> colsum_fused;
@@ -685,7 +685,7 @@ void Executor::build() {
   std::set<uint32_t> folded_scalar;
 
   // Mixed precision: every value a GEMM reads as an operand gets an f16 copy in HBM, which the
-  // f16 GEMM (k_gemm_lds16) reads straight into LDS: a GEMM output's copy is written by the GEMM's
+  // f16 GEMM (gemm16) reads straight into LDS: a GEMM output's copy is written by the GEMM's
   // epilogue, a LayerNorm's (forward or backward) by the LayerNorm pass, a parameter's by the
   // optimizer launch (and every upload); other producers (attention, cross-entropy) are followed by
   // a rounding pass. The f32 values stay for the kernels that read them in f32.
@@ -854,6 +854,7 @@ void Executor::build() {
     float drop_scale = 1.0f;
     // Further K segments (A, B sources) of a chain of like GEMMs added into one value.
     std::vector<std::pair<uint32_t, uint32_t>> segs;
+    std::vector<uint32_t> merged;  // the MatMul nodes of a chain merged into this job, itself aside
     std::string what;
     bool c16 = false;  // mixed precision: the output's f16 copy is written too
     // Mixed precision: false for an operand or output held only as its f16 copy.
@@ -925,9 +926,13 @@ void Executor::build() {
                           a.ksegs = int(1 + j.segs.size());
                           a.seg_a[0] = a.a;
                           a.seg_b[0] = a.b;
+                          a.seg_a16[0] = a.h16 ? ptr16(j.asrc) : nullptr;
+                          a.seg_b16[0] = a.h16 ? ptr16(j.bsrc) : nullptr;
                           for (size_t t = 0; t < j.segs.size(); ++t) {
-                            a.seg_a[t + 1] = F(j.segs[t].first);
-                            a.seg_b[t + 1] = F(j.segs[t].second);
+                            a.seg_a[t + 1] = a.h16 ? nullptr : F(j.segs[t].first);
+                            a.seg_b[t + 1] = a.h16 ? nullptr : F(j.segs[t].second);
+                            a.seg_a16[t + 1] = a.h16 ? ptr16(j.segs[t].first) : nullptr;
+                            a.seg_b16[t + 1] = a.h16 ? ptr16(j.segs[t].second) : nullptr;
                           }
                         }
                         if (j.epi.node != j.id && j.epi.act == hk::EPI_NONE) a.addend = F(uint32_t(j.epi.aux));
@@ -1851,11 +1856,17 @@ void Executor::build() {
   // GEMM's place. The sum is one contraction instead of n rounded partial products: within the
   // per-kernel tolerance of the reference's order, not bit-identical to it. (The backward of the
   // Q, K and V projections: the three input gradients added into the residual gradient.)
+  // Under mixed precision the segments are read as f16 copies by gemm16, K tiles of 64 (BERT-base's
+  // three 16384 x 768 x 768 products, each adding 50 MB of f32 into the next: 3 x 42 us, in one 65).
   {
+    auto has16 = [&](uint32_t v) {
+      return token16_.count(v) || fixed16_.count(v) || (s_.opt_.plan_only && p.node(v).op == Op::ParamRead);
+    };
     auto chainable = [&](const GemmJob& j) {
       return j.epi.node != j.id && j.epi.act == hk::EPI_NONE && j.bias_id < 0 && j.cs_id < 0 && !j.ws &&
-             !j.ce_part && !j.ce_tab && j.segs.empty() && !j.g.defer && !j.g.h16 && j.g.k % 32 == 0 &&
-             hk::gemm_split_for(j.g.m, j.g.n, j.g.k, false, j.g.h16) == 1;
+             !j.ce_part && !j.ce_tab && j.segs.empty() && !j.g.defer &&
+             (j.g.h16 ? mixed_twins && j.g.k % 64 == 0 && has16(j.asrc) && has16(j.bsrc) && hk::gemm16_fits(j.g)
+                      : j.g.k % 32 == 0);
     };
     auto same = [](const hk::GemmArgs& a, const hk::GemmArgs& b) {
       return a.m == b.m && a.n == b.n && a.k == b.k && a.lda == b.lda && a.ldb == b.ldb && a.ldc == b.ldc &&
@@ -1871,6 +1882,7 @@ void Executor::build() {
       while (chain.size() < size_t(hk::kGemmGroupMax)) {
         const GemmJob& cur = *pending[chain.back()].gemm[0];
         if (cur.epi.drop >= 0 || consumers[p.pos.at(cur.out_id)].size() != 1) break;
+        if (hk::gemm_split_for(head.g.m, head.g.n, head.g.k * int64_t(chain.size() + 1), false, head.g.h16) != 1) break;
         size_t nxt = SIZE_MAX;
         for (size_t j = chain.back() + 1; j < pending.size() && nxt == SIZE_MAX; ++j)
           if (!gone[j] && pending[j].gemm.size() == 1 && !pending[j].side && chainable(*pending[j].gemm[0]) &&
@@ -1891,6 +1903,7 @@ void Executor::build() {
       merged.bytes = 0;
       for (size_t c = 0; c < chain.size(); ++c) {
         const GemmJob& m = *pending[chain[c]].gemm[0];
+        if (c + 1 < chain.size()) job->merged.push_back(m.id);
         if (c > 0) {
           job->segs.push_back({m.asrc, m.bsrc});
           job->what += " (+) " + m.what.substr(m.what.find('%'));
@@ -1986,8 +1999,8 @@ void Executor::build() {
     }
     pending = std::move(merged);
   }
-  // Mixed precision: a GEMM output that only k_gemm_lds16 launches read (as operands, or the
-  // column sums they take) is kept as its f16 copy alone: its producer (itself on k_gemm_lds16)
+  // Mixed precision: a GEMM output that only gemm16 launches read (as operands, or the
+  // column sums they take) is kept as its f16 copy alone: its producer (itself on gemm16)
   // writes no f32 value, and its readers get no f32 pointer for it, so that any other kernel
   // refuses the problem loudly.
   if (mixed_twins && !s_.opt_.plan_only) {
@@ -1995,14 +2008,17 @@ void Executor::build() {
     std::map<uint32_t, GemmJob*> job_of;   // MatMul node -> its GEMM job
     std::map<int64_t, GemmJob*> sums_of;  // fused SumRows node -> its GEMM job
     std::map<uint32_t, GemmJob*> producer;
-    std::set<const GemmJob*> certain;     // jobs whose launch runs k_gemm_lds16
+    std::set<const GemmJob*> certain;     // jobs whose launch runs gemm16
     for (auto& pd : pending) {
       bool all = !pd.gemm.empty();
-      for (auto& j : pd.gemm)
-        all = all && j->segs.empty() && has16(j->asrc) && has16(j->bsrc) && hk::gemm_lds16_fits(j->g);
+      for (auto& j : pd.gemm) {
+        all = all && has16(j->asrc) && has16(j->bsrc) && hk::gemm16_fits(j->g);
+        for (auto& sg : j->segs) all = all && has16(sg.first) && has16(sg.second);
+      }
       for (auto& j : pd.gemm) {
         const Node& jn = p.node(j->id);
         job_of[jn.op == Op::AddRows ? jn.operands[0] : j->id] = j.get();
+        for (uint32_t mid : j->merged) job_of[mid] = j.get();
         if (j->cs_id >= 0) sums_of[j->cs_id] = j.get();
         producer[j->out_id] = j.get();
         if (all) certain.insert(j.get());
@@ -2036,7 +2052,9 @@ void Executor::build() {
         if (c.op == Op::SumRows && sums_of.count(c.id)) j = sums_of.at(c.id);
         if (!j || !certain.count(j) || j->bias_id == int64_t(v) || (j->epi.node != j->id && j->epi.aux == int64_t(v)))
           return false;
-        if (j->asrc != v && j->bsrc != v) return false;
+        bool reads = j->asrc == v || j->bsrc == v;
+        for (auto& sg : j->segs) reads = reads || sg.first == v || sg.second == v;
+        if (!reads) return false;
       }
       return !readers.empty();
     };

@@ -49,3 +49,99 @@ def test_attention_over_partial_tiles(ctx, oracle, B, L, S, H, heads, mixed):
         assert ok, (idx, worst)
     for g in (got[2], got[3]):
         assert np.all(g.reshape(B * S, H)[mask.reshape(-1) == 0] == 0)
+
+
+def f16(x):
+    return np.asarray(x, np.float32).astype(np.float16).astype(np.float64)
+
+
+@pytest.fixture
+def mixed(ctx):
+    ctx.set_precision(True)
+    yield ctx
+    ctx.set_precision(False)
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("m,k,n", [
+    (8000, 72, 1496),   # 256 x 192 tiles (128 x 128 for both operands transposed), a K tail of 8
+    (2000, 136, 2104),  # 128 x 128 tiles, partial ones at both edges, a K tail of 8
+    (1000, 520, 1096),  # 64 x 64 tiles
+    (1000, 24, 1096),   # one partial K tile
+    (72, 1032, 88),     # 64 x 32 tiles, a K tail of 8
+    (8, 256, 8),        # one partial tile
+    (296, 9000, 200),   # split-K slices and their sum
+])
+def test_mixed_gemm_tiles(mixed, m, k, n, ta, tb):
+    """Every tile of the f16 GEMM at partial tiles and K tails, against the float64 product of the
+    f16 operands (1e-5 of the sum of |terms|, f32 accumulation)."""
+    rng = np.random.default_rng(m + k)
+    a = rng.standard_normal((k, m) if ta else (m, k)).astype(np.float32)
+    b = rng.standard_normal((n, k) if tb else (k, n)).astype(np.float32)
+    p = Prog()
+    ai, bi = p.input("a", a.shape), p.input("b", b.shape)
+    lhs = p.op("Transpose", [ai], (m, k)) if ta else ai
+    rhs = p.op("Transpose", [bi], (k, n)) if tb else bi
+    p.out(p.op("MatMul", [lhs, rhs], (m, n)))
+    prog = mixed.program(p.text())
+    prog.run({"a": a, "b": b})
+    got = prog.output(0, m * n).reshape(m, n)
+    A, Bm = f16(a.T if ta else a), f16(b.T if tb else b)
+    bound = 1e-5 * (np.abs(A) @ np.abs(Bm)) + 1e-30
+    worst = np.max(np.abs(got - A @ Bm) / bound)
+    assert worst <= 1.0, worst
+
+
+@pytest.mark.parametrize("rows,h,f", [(64, 64, 256), (2048, 256, 1024), (4096, 320, 1280), (304, 96, 392)])
+def test_mixed_ffn_on_f16_values(mixed, rows, h, f):
+    """gelu(x w1 + b1) w2 and its input gradient, the GELU's output and the pre-activation held as
+    f16: each result within 2^-9 of the sum of |terms| of the float64 value, i.e. one f16 rounding
+    (2^-11) of each factor of its last product and of the values behind it."""
+    rng = np.random.default_rng(rows)
+    x, dy = (rng.standard_normal((rows, h)).astype(np.float32) for _ in range(2))
+    w1 = (rng.standard_normal((h, f)) / np.sqrt(h) * 2).astype(np.float32)
+    w2 = (rng.standard_normal((f, h)) / np.sqrt(f)).astype(np.float32)
+    b1 = rng.standard_normal(f).astype(np.float32)
+    p = Prog()
+    xi, gi, w1i, w2i = p.input("x", x.shape), p.input("dy", dy.shape), p.input("w1", w1.shape), p.input("w2", w2.shape)
+    bi = p.input("b1", b1.shape)
+    pre = p.op("AddRows", [p.op("MatMul", [xi, w1i], (rows, f)), bi], (rows, f))
+    y = p.op("MatMul", [p.op("Gelu", [pre], (rows, f)), w2i], (rows, h))
+    dg = p.op("MatMul", [gi, p.op("Transpose", [w2i], (h, f))], (rows, f))
+    dx = p.op("MatMul", [p.op("GeluGrad", [pre, dg], (rows, f)), p.op("Transpose", [w1i], (f, h))], (rows, h))
+    p.out(y, dx)
+    prog = mixed.program(p.text())
+    prog.run({"x": x, "dy": dy, "w1": w1, "w2": w2, "b1": b1})
+    got_y, got_dx = (prog.output(k, rows * h).reshape(rows, h) for k in (0, 1))
+    u = f16(x) @ f16(w1) + b1
+    t = np.tanh(np.sqrt(2 / np.pi) * (u + 0.044715 * u ** 3))
+    gelu = 0.5 * u * (1 + t)
+    slope = 0.5 * (1 + t) + 0.5 * u * (1 - t * t) * np.sqrt(2 / np.pi) * (1 + 3 * 0.044715 * u * u)
+    gated = (f16(dy) @ f16(w2).T) * slope
+    for got, left, right in ((got_y, gelu, f16(w2)), (got_dx, gated, f16(w1).T)):
+        bound = 2.0 ** -9 * ((np.abs(left) + 0.02) @ np.abs(right))
+        worst = np.max(np.abs(got - left @ right) / bound)
+        assert worst <= 1.0, worst
+
+
+@pytest.mark.parametrize("rows,h", [(200, 64), (4096, 192), (16, 320), (1000, 96)])
+def test_mixed_chains_of_products(mixed, rows, h):
+    """x + a1 w1 + a2 w2 + a3 w3, each product read only by the next sum: one product over the
+    concatenated K where h is a multiple of 64, separate ones (h = 96) otherwise."""
+    rng = np.random.default_rng(h)
+    x, a1, a2, a3 = (rng.standard_normal((rows, h)).astype(np.float32) for _ in range(4))
+    w1, w2, w3 = (rng.standard_normal((h, h)).astype(np.float32) for _ in range(3))
+    p = Prog()
+    xi = p.input("x", (rows, h))
+    total = xi
+    for k in (1, 2, 3):
+        ai, wi = p.input(f"a{k}", (rows, h)), p.input(f"w{k}", (h, h))
+        total = p.op("Add", [total, p.op("MatMul", [ai, p.op("Transpose", [wi], (h, h))], (rows, h))], (rows, h))
+    p.out(total)
+    prog = mixed.program(p.text())
+    prog.run({"x": x, "a1": a1, "a2": a2, "a3": a3, "w1": w1, "w2": w2, "w3": w3})
+    got = prog.output(0, rows * h).reshape(rows, h)
+    want, mag = x.astype(np.float64), np.abs(x).astype(np.float64)
+    for a, w in ((a1, w1), (a2, w2), (a3, w3)):
+        want, mag = want + f16(a) @ f16(w).T, mag + np.abs(f16(a)) @ np.abs(f16(w)).T
+    assert np.max(np.abs(got - want) / mag) <= 1e-5
