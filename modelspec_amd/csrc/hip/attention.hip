@@ -1136,20 +1136,26 @@ bool bwd_fits(int64_t L, int64_t S, int64_t d) {
 bool head_ok(int64_t d) { return d == 16 || d == 32 || d == 64 || d == 128; }
 // The streaming shape, from measured MI355X timings: problems of 4096 or more 16-row wave tiles
 // (BERT-base: 12288) take blocks of four waves and tiles of 32 rows (35 KB of LDS a block at
-// D = 64, four blocks a CU); smaller ones (BERT-tiny: 512) blocks of two waves and tiles of 64
-// rows (32 for D = 128), so that the few waves spread over more CUs with longer MFMA chains.
+// D = 64, four blocks a CU); smaller ones blocks of two waves and tiles of 64 rows (f16; 32 rows for
+// D = 128), so that the few waves spread over more CUs with longer MFMA chains.
 // ks: waves sharing a row tile (each a share of every streamed tile); one: the streamed side fits
 // one tile, so one LDS buffer and no prefetch. Small problems whose streamed side is at most 128
 // rows (BERT-tiny: 512 wave tiles on 1024 SIMDs) take one 128-row tile shared by two waves a row
 // tile, twice the waves (f32 only; on BERT-tiny the backward pair went from 34 to 27 us a layer
 // and the step from 0.955 to 0.935 ms; four waves a row tile in blocks of eight took the forward
 // from 10.0 to 11.3 us and the backward from 21.3 to 32.4 us).
+// Longer f32 sequences of heads up to 64 wide in between (8 x 512 rows, 4 heads: 1024 wave tiles on 1024
+// SIMDs): the forward two waves a row tile on 64-row tiles, the backward 32-row tiles, so that a CU
+// holds 8 and 16 waves instead of 4 (us a layer, one wave a row tile on 64-row tiles before: forward
+// 62.5 -> 39.6, backward 174.7 -> 92.7; 8 x 256 rows: 22.0 -> 15.9, 45.7 -> 35.6; the backward on
+// the forward's plan 106 and 34, the forward on the backward's 44.7 and 24.2).
 struct AttnPlan { int T, W, KS; bool one; };
-AttnPlan attn_plan(int64_t bh, int64_t rows, int64_t streamed, int64_t d, bool h16) {
+AttnPlan attn_plan(int64_t bh, int64_t rows, int64_t streamed, int64_t d, bool h16, bool forward) {
   const int64_t tiles = bh * ((rows + 15) / 16);
   AttnPlan p;
   if (tiles >= 4096) p = {32, 4, 1, false};
   else if (!h16 && streamed <= 128 && d <= 64) p = {128, 4, 2, false};
+  else if (!h16 && d <= 64) p = forward ? AttnPlan{64, 4, 2, false} : AttnPlan{32, 4, 1, false};
   else p = {d >= 128 ? 32 : 64, 2, 1, false};
   p.one = streamed <= p.T;
   return p;
@@ -1217,7 +1223,6 @@ void launch_bwd(hipStream_t s, dim3 grid, unsigned qy, bool one, const float* q,
   } else {                                                 \
     if ((plan).KS == 2) GO_F(128, 4, 2);                   \
     else if ((plan).W == 4) GO_F(32, 4, 1);                \
-    else if ((plan).T == 64) GO_F(64, 2, 1);               \
     else GO_F(32, 2, 1);                                   \
   }
 }  // namespace
@@ -1248,12 +1253,17 @@ void attention_fwd(hipStream_t s, const float* q, const float* k, const float* v
     MSX_LAUNCH(k_attn_fwd_reg<4>, grid, dim3(256), 0, s, q, k, v, mask, o, stats, int(L), int(H), int(heads), scale);
     return;
   }
-  const AttnPlan plan = attn_plan(B * heads, L, S, d, h16);
+  const AttnPlan plan = attn_plan(B * heads, L, S, d, h16, true);
   dim3 grid(unsigned(B * heads), row_blocks(L, plan));
 #define GO_H(T, W) launch_fwd_h<D, T, W>(s, grid, q, k, v, mask, o, stats, int(L), int(S), int(H), int(heads), scale)
 #define GO_F(T, W, KS) \
   launch_fwd<D, T, W, KS>(s, grid, plan.one, q, k, v, mask, o, stats, int(L), int(S), int(H), int(heads), scale)
-#define GO(D_) { constexpr int D = D_; MSX_BY_PLAN(plan, h16, GO_H, GO_F) }
+#define GO(D_)                                                 \
+  {                                                            \
+    constexpr int D = D_;                                      \
+    if (D <= 64 && plan.T == 64 && plan.KS == 2) GO_F(64, 4, 2); \
+    else MSX_BY_PLAN(plan, h16, GO_H, GO_F)                    \
+  }
   MSX_BY_D(d, GO)
 #undef GO
 #undef GO_F
@@ -1270,7 +1280,7 @@ void attention_bwd(hipStream_t s, const float* q, const float* k, const float* v
   h16 = h16 && whole_tiles(L, S);
   if (!o || !stats || !dsum) refuse("the MFMA attention backward needs the forward output and statistics");
   if (!dq) refuse("the MFMA attention backward computes d_i in its dQ pass: dQ is required");
-  const AttnPlan pq = attn_plan(B * heads, L, S, d, h16);
+  const AttnPlan pq = attn_plan(B * heads, L, S, d, h16, false);
   dim3 gq(unsigned(B * heads), row_blocks(L, pq));
   if (!h16 && dk && dv && L == S) {
     // Self-attention in f32: one launch for both passes (the key pass plans as the query pass).
@@ -1297,7 +1307,7 @@ void attention_bwd(hipStream_t s, const float* q, const float* k, const float* v
 #undef GO_F
 #undef GO_H
   if (dk || dv) {
-    const AttnPlan pk = attn_plan(B * heads, S, L, d, h16);
+    const AttnPlan pk = attn_plan(B * heads, S, L, d, h16, false);
     dim3 gk(unsigned(B * heads), row_blocks(S, pk));
 #define GO_H(T, W) \
   launch_bwd_kv_h<D, T, W>(s, gk, q, k, v, mask, stats, g, dsum, dk, dv, int(L), int(S), int(H), int(heads), scale)
@@ -1316,6 +1326,7 @@ void prepare_attention() {
   const void* kernels[] = {
 #define MSX_ATTN_W(D, T, W)                                         \
   reinterpret_cast<const void*>(k_attn_fwd_mfma<D, T, W>),          \
+      reinterpret_cast<const void*>(k_attn_fwd_mfma<D, 64, 4, 2>),  \
       reinterpret_cast<const void*>(k_attn_bwd_q_mfma<D, T, W>),    \
       reinterpret_cast<const void*>(k_attn_bwd_kv_mfma<D, T, W>),   \
       reinterpret_cast<const void*>(k_attn_fwd_mfma<D, 128, 4, 2>), \
@@ -1328,7 +1339,7 @@ void prepare_attention() {
       reinterpret_cast<const void*>(k_attn_bwd_q_h16<D, T, W>),     \
       reinterpret_cast<const void*>(k_attn_bwd_kv_h16<D, T, W>)
 #define MSX_ATTN_K(D)                                                                            \
-  MSX_ATTN_W(D, 32, 4), MSX_ATTN_W(D, 64, 2), MSX_ATTN_W(D, 32, 2), MSX_ATTN_H(D, 32, 4), \
+  MSX_ATTN_W(D, 32, 4), MSX_ATTN_W(D, 32, 2), MSX_ATTN_H(D, 32, 4), \
       MSX_ATTN_H(D, 64, 2), MSX_ATTN_H(D, 32, 2)
       MSX_ATTN_K(16), MSX_ATTN_K(32), MSX_ATTN_K(64), MSX_ATTN_K(128)};
 #undef MSX_ATTN_K

@@ -382,7 +382,7 @@ __global__ __launch_bounds__(256) void k_gemm_w(GemmPtrs ptrs, int64_t M, int64_
             smem[(wm - pass * PR + 16 * i + 4 * (lane >> 4) + r) * LC + wn + 16 * j + (lane & 15)] = acc[i][j][r];
     }
     __syncthreads();
-#pragma unroll
+#pragma unroll 1
     for (int e0 = 0; e0 < PR * Q; e0 += 256) {
       const int e = e0 + tid;
       if (PR * Q % 256 != 0 && e >= PR * Q) break;
@@ -419,14 +419,13 @@ __global__ __launch_bounds__(256) void k_gemm_w(GemmPtrs ptrs, int64_t M, int64_
         *reinterpret_cast<float4*>(out + row * ldo + col) = ws ? v : gemm_epilogue4(epi, v, row, col, ldo);
       } else if (vo && col < N) {
         // The last group of a row padded to a multiple of 4: zeros in the padding.
-        const float vs[4] = {v.x, v.y, v.z, v.w};
-        float r4[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) r4[c] = col + c < N ? (ws ? vs[c] : gemm_epilogue(epi, vs[c], row, col + c, ldo)) : 0.0f;
-        *reinterpret_cast<float4*>(out + row * ldo + col) = make_float4(r4[0], r4[1], r4[2], r4[3]);
+        const float* vs = smem + rl * LC + c4;
+#pragma unroll 1
+        for (int c = 0; c < 4; ++c)
+          out[row * ldo + col + c] = col + c < N ? (ws ? vs[c] : gemm_epilogue(epi, vs[c], row, col + c, ldo)) : 0.0f;
       } else {
-        const float vs[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
+        const float* vs = smem + rl * LC + c4;
+#pragma unroll 1
         for (int c = 0; c < 4; ++c)
           if (col + c < N) out[row * ldo + col + c] = ws ? vs[c] : gemm_epilogue(epi, vs[c], row, col + c, ldo);
       }

@@ -64,7 +64,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_lds(GemmPtrs ptrs, int6
   const float* __restrict__ bias = epi.bias;
   float* __restrict__ ws = ptrs.ws[0];
   float* __restrict__ colsum = ptrs.colsum[0];
-  auto fsw = [](int r) { return BK == 16 ? (r >> 2) & 3 : (r >> 1) & 7; };
+  auto fsw = [](int r) { return BK == 16 ? -(r >> 2) & 3 : (r >> 1) & 7; };
   // Each load instruction's per-lane source at the slice's first K tile. KC: instruction t holds
   // rows t RPI .. (lane L: row L / LPR, K group (L % LPR) ^ f(row)). Not KC: K rows t (256 / R) ..
   // of R = BM (BN) floats (lane L: rows 4 (L % (R / 4)) .. + 3 at K row L / (R / 4)); the last

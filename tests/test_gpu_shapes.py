@@ -35,10 +35,14 @@ def attention_case(ctx, oracle, B, L, S, H, heads):
     (3, 300, 300, 32, 2),    # several streamed tiles, the last of 44 rows
     (43, 100, 100, 224, 14),  # over 4096 row tiles: four-wave blocks streaming 32-row tiles
     (2, 20, 48, 64, 2),      # fewer queries than keys, whole key tiles
+    (2, 528, 528, 128, 2),   # long sequences: 64-row tiles forward, 32-row backward, partial last ones
+    (1, 140, 144, 64, 1),    # the shortest of these, fewer queries than keys
 ])
 def test_attention_over_partial_tiles(ctx, oracle, B, L, S, H, heads, mixed):
-    """Row counts that are no multiple of 16, in f32 also under mixed precision: rows past the end
-    take no part and are not written, masked keys' gradients are +0."""
+    """Partial tiles of rows, in f32 (also under mixed precision where a row count is no multiple of 16):
+    rows past the end take no part and are not written, masked keys' gradients are +0."""
+    if mixed and L % 16 == 0 and S % 16 == 0:
+        pytest.skip("whole tiles under mixed precision are the f16 kernels', tested with them")
     ctx.set_precision(mixed)
     try:
         got, want, mask, scale = attention_case(ctx, oracle, B, L, S, H, heads)
