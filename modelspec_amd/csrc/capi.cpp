@@ -80,6 +80,18 @@ msx::Batch batch_of(const msx_tensor* t, uint32_t n) {
   }
   return b;
 }
+
+// The same without a copy: the caller's memory, valid during the call.
+msx::BatchView view_of(const msx_tensor* t, uint32_t n) {
+  msx::BatchView b;
+  for (uint32_t i = 0; i < n; ++i) {
+    if (!t[i].name) throw msx::IrError("an input has no name");
+    if (t[i].dtype == 0) b.f32[t[i].name] = {static_cast<const float*>(t[i].data), size_t(t[i].count)};
+    else if (t[i].dtype == 1) b.i32[t[i].name] = {static_cast<const int32_t*>(t[i].data), size_t(t[i].count)};
+    else throw msx::IrError(std::string("input `") + t[i].name + "` has an unknown dtype");
+  }
+  return b;
+}
 }  // namespace
 
 struct msx_ctx {
@@ -106,16 +118,17 @@ msx::SessionOptions config_options(const msx_ctx* ctx, const msx::Compiled& c) {
 }
 
 // With a corpus loaded, a batch that names `data.step` (i32 [low, high] of the step) is the
-// corpus batch of that step: its sequences are drawn here and the device draws its rows.
-void corpus_draw(msx_ctx* ctx, msx::Batch& b, msx::SplitRole role) {
+// corpus batch of that step: its sequences are drawn here (into `words`, which the view then reads)
+// and the device draws its rows.
+void corpus_draw(msx_ctx* ctx, msx::BatchView& b, msx::SplitRole role, std::vector<int32_t>& words) {
   auto it = b.i32.find("data.step");
   if (it == b.i32.end()) return;
   if (!ctx->corpus || !ctx->session) throw msx::IrError("`data.step` names a corpus batch, and no corpus is loaded");
   if (it->second.size() != 2) throw msx::IrError("`data.step` is i32 [low, high]");
   const uint64_t step = uint64_t(uint32_t(it->second[0])) | (uint64_t(uint32_t(it->second[1])) << 32);
   b.i32.erase(it);
-  b.i32[msx::kDrawInput] =
-      msx::draw_words(role, ctx->orders.draw(*ctx->corpus, role, ctx->seed, step, ctx->session->corpus_batch()));
+  words = msx::draw_words(role, ctx->orders.draw(*ctx->corpus, role, ctx->seed, step, ctx->session->corpus_batch()));
+  b.i32[msx::kDrawInput] = {words.data(), words.size()};
 }
 }  // namespace
 
@@ -226,9 +239,7 @@ int msx_set_params(msx_ctx* ctx, const float* const* values, const uint64_t* cou
 int msx_read_param(msx_ctx* ctx, uint32_t param, float* out, uint64_t count) {
   return guarded([&] {
     if (!ctx->session) return fail(MSX_E_INVALID, "no step is loaded");
-    auto all = ctx->session->params();
-    if (param >= all.size() || all[param].size() != count) return fail(MSX_E_INVALID, "no such parameter or wrong count");
-    std::memcpy(out, all[param].data(), count * 4);
+    if (!ctx->session->read_param(param, 'p', out, count)) return fail(MSX_E_INVALID, "no such parameter or wrong count");
     return MSX_OK;
   });
 }
@@ -236,9 +247,8 @@ int msx_read_param(msx_ctx* ctx, uint32_t param, float* out, uint64_t count) {
 int msx_read_moment(msx_ctx* ctx, uint32_t param, int32_t which, float* out, uint64_t count) {
   return guarded([&] {
     if (!ctx->session) return fail(MSX_E_INVALID, "no step is loaded");
-    auto all = ctx->session->moments(char(which));
-    if (param >= all.size() || all[param].size() != count) return fail(MSX_E_INVALID, "no such moment or wrong count");
-    std::memcpy(out, all[param].data(), count * 4);
+    if (!ctx->session->read_param(param, which == 'm' ? 'm' : 'v', out, count))
+      return fail(MSX_E_INVALID, "no such moment or wrong count");
     return MSX_OK;
   });
 }
@@ -246,18 +256,18 @@ int msx_read_moment(msx_ctx* ctx, uint32_t param, int32_t which, float* out, uin
 int msx_run_steps(msx_ctx* ctx, uint32_t n, const msx_tensor* const* inputs, const uint32_t* n_inputs, float* losses_out) {
   return guarded([&] {
     if (!ctx->session) return fail(MSX_E_INVALID, "no step is loaded");
-    size_t before = ctx->session->losses().size();
+    const size_t before = ctx->session->logged();
+    std::vector<int32_t> words;
     for (uint32_t i = 0; i < n; ++i) {
-      msx::StepInputs in;
-      in.batch = batch_of(inputs[i], n_inputs[i]);
-      corpus_draw(ctx, in.batch, msx::SplitRole::Train);
-      ctx->session->train_step(in);
+      msx::BatchView in = view_of(inputs[i], n_inputs[i]);
+      corpus_draw(ctx, in, msx::SplitRole::Train, words);
+      ctx->session->run_step(in);
     }
-    auto all = ctx->session->losses();
+    auto logged = ctx->session->losses_from(before);
     if (losses_out)
-      for (uint32_t i = 0; i < n; ++i) losses_out[i] = all.at(before + i);
+      for (uint32_t i = 0; i < n; ++i) losses_out[i] = logged.at(i);
     for (uint32_t i = 0; i < n; ++i)
-      if (!std::isfinite(all.at(before + i)))
+      if (!std::isfinite(logged.at(i)))
         return fail(MSX_E_NONFINITE, "E-TRAIN-001: the loss of step " + std::to_string(before + i) + " is not finite");
     return MSX_OK;
   });
@@ -267,9 +277,10 @@ int msx_forward(msx_ctx* ctx, const msx_tensor* inputs, uint32_t n_inputs, float
                 uint64_t prediction_count) {
   return guarded([&] {
     if (!ctx->session) return fail(MSX_E_INVALID, "no step is loaded");
-    msx::Batch b = batch_of(inputs, n_inputs);
-    corpus_draw(ctx, b, msx::SplitRole::Train);
-    float loss = ctx->session->final_loss(b);
+    msx::BatchView b = view_of(inputs, n_inputs);
+    std::vector<int32_t> words;
+    corpus_draw(ctx, b, msx::SplitRole::Train, words);
+    float loss = ctx->session->forward_loss(b);
     if (loss_out) *loss_out = loss;
     if (prediction_out) {
       const uint32_t pred = ctx->prediction;
@@ -755,7 +766,7 @@ int msx_prog_run(msx_prog* prog, const msx_tensor* inputs, uint32_t n_inputs, co
     std::vector<std::vector<float>> v;
     for (uint32_t i = 0; i < n_params; ++i) v.emplace_back(params[i], params[i] + param_counts[i]);
     prog->session->load_params(v);
-    prog->session->run_forward(batch_of(inputs, n_inputs));
+    prog->session->run_forward(view_of(inputs, n_inputs));
     return MSX_OK;
   });
 }

@@ -2256,7 +2256,7 @@ std::string Executor::plan_text() const {
   return out;
 }
 
-void Executor::stage(const Batch& batch) {
+void Executor::stage(const BatchView& batch) {
   auto fed = [&](const std::string& name) {
     for (auto& in : inputs_)
       if (in.device && in.name == name) return true;
@@ -2530,7 +2530,7 @@ const void* Session::step_value(uint32_t id) const {
   return step_exec_->value(id);
 }
 
-void Session::run_forward(const Batch& batch) {
+void Session::run_forward(const BatchView& batch) {
   fwd_exec_->stage(batch);
   fwd_exec_->run(stream_);
   sync();
@@ -2610,8 +2610,8 @@ std::vector<float> Session::predict(const std::vector<std::vector<float>>& value
   return out;
 }
 
-void Session::train_step(const StepInputs& in) {
-  step_exec_->stage(in.batch);
+void Session::run_step(const BatchView& batch) {
+  step_exec_->stage(batch);
   if (use_graph_) {
     if (!graph_exec_) {
       hip_check(hipStreamBeginCapture(stream_, hipStreamCaptureModeRelaxed), "hipStreamBeginCapture");
@@ -2680,7 +2680,7 @@ std::vector<Session::Timed> Session::profile_step(const StepInputs& in) {
   return out;
 }
 
-float Session::final_loss(const Batch& batch) {
+float Session::forward_loss(const BatchView& batch) {
   fwd_exec_->stage(batch);
   fwd_exec_->run(stream_);
   sync();
@@ -2758,15 +2758,32 @@ std::string Session::plan_text() const {
   return out;
 }
 
-std::vector<float> Session::losses() {
+size_t Session::logged() {
   sync();
   uint32_t count = 0;
   hip_check(hipMemcpy(&count, counter_, 4, hipMemcpyDeviceToHost), "hipMemcpy (loss counter)");
   check_data_error();
-  count = std::min(count, loss_capacity_);
-  std::vector<float> out(count);
-  if (count) hip_check(hipMemcpy(out.data(), losses_dev_, count * 4, hipMemcpyDeviceToHost), "hipMemcpy (losses)");
+  return std::min(count, loss_capacity_);
+}
+
+std::vector<float> Session::losses_from(size_t first) {
+  const size_t count = logged();
+  std::vector<float> out(count > first ? count - first : 0);
+  if (!out.empty())
+    hip_check(hipMemcpy(out.data(), losses_dev_ + first, out.size() * 4, hipMemcpyDeviceToHost), "hipMemcpy (losses)");
   return out;
+}
+
+bool Session::read_param(uint32_t param, char which, float* out, uint64_t count) {
+  const auto& params = step_.program.params;
+  if (param >= params.size()) return false;
+  const bool held = which == 'p' || step_.moments.count(param);  // an SGD step holds no moments
+  if (uint64_t(held ? params[param].ty.count() : 0) != count) return false;
+  sync();
+  const float* base = which == 'm' ? m_ : which == 'v' ? v_ : param_;
+  if (count)
+    hip_check(hipMemcpy(out, base + offset_[param], count * 4, hipMemcpyDeviceToHost), "hipMemcpy (read parameter)");
+  return true;
 }
 
 }  // namespace msx

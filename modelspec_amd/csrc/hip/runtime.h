@@ -62,6 +62,26 @@ struct RunStats {
   uint64_t steps = 0, graph_launches = 0, kernels_per_step = 0, bytes_uploaded = 0, device_bytes = 0;
 };
 
+// The inputs of one step or forward pass where the caller holds them: named f32 and i32 spans, read
+// while they are staged.
+struct BatchView {
+  template <class T>
+  struct Span {
+    const T* p = nullptr;
+    size_t n = 0;
+    const T* data() const { return p; }
+    size_t size() const { return n; }
+    const T& operator[](size_t i) const { return p[i]; }
+  };
+  std::map<std::string, Span<float>> f32;
+  std::map<std::string, Span<int32_t>> i32;
+  BatchView() = default;
+  BatchView(const Batch& b) {
+    for (auto& [name, v] : b.f32) f32[name] = {v.data(), v.size()};
+    for (auto& [name, v] : b.i32) i32[name] = {v.data(), v.size()};
+  }
+};
+
 class Executor;
 
 // A loaded training run on one device.
@@ -94,8 +114,16 @@ class Session : public Engine {
   std::vector<std::vector<float>> moments(char which) override;
   void set_moments(const std::vector<std::vector<float>>& m, const std::vector<std::vector<float>>& v) override;
   std::vector<float> predict(const std::vector<std::vector<float>>& values, const Batch& batch) override;
-  void train_step(const StepInputs& in) override;
-  float final_loss(const Batch& batch) override;
+  void train_step(const StepInputs& in) override { run_step(in.batch); }
+  void run_step(const BatchView& batch);
+  float final_loss(const Batch& batch) override { return forward_loss(batch); }
+  float forward_loss(const BatchView& batch);
+  // One parameter ('p'), or its first ('m') or second ('v') moment, straight into the caller's
+  // memory; false where it does not exist or has another size.
+  bool read_param(uint32_t param, char which, float* out, uint64_t count);
+  // Losses logged so far, and those from the `first` on.
+  size_t logged();
+  std::vector<float> losses_from(size_t first);
   // The forward program over every held-out batch, each batch's logits reduced on the device to
   // the row losses and hits (held_out_rows) and added into one f64 sum and one count
   // (held_out_sum); one host wait at the end (vulkan/stepwise.rs:1635-1760 does the same with its
@@ -106,7 +134,7 @@ class Session : public Engine {
   // every call on one device shares the array, so calls that overlap on a device race.
   HeldOutSums held_out_static(const HeldOut& h);
   static constexpr int64_t kStaticEvalRows = 65536;
-  std::vector<float> losses() override;
+  std::vector<float> losses() override { return losses_from(0); }
   // The plans of a plan-only (or any) session: the step's, then the forward program's.
   std::string plan_text() const;
 
@@ -121,7 +149,7 @@ class Session : public Engine {
   const RunStats& stats() const { return stats_; }
   size_t launches_per_step() const;
   // The forward program alone, on the current parameters (per-op tests, evaluation).
-  void run_forward(const Batch& batch);
+  void run_forward(const BatchView& batch);
   const void* forward_value(uint32_t id) const;
   // A value of the step program (its inputs among them) as the last step left it.
   const void* step_value(uint32_t id) const;
@@ -198,7 +226,7 @@ class Executor {
   ~Executor();
   // Packs `batch` (and checks ids, labels and key masks) into the next pinned slot and enqueues
   // its copy to the device input block.
-  void stage(const Batch& batch);
+  void stage(const BatchView& batch);
   void run(hipStream_t s);  // every launch, in order
   const std::vector<Launch>& launches() const { return launches_; }
   // The launch plan as text: one line a launch (its place, the values it completes, side stream,
