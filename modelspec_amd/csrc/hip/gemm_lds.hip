@@ -30,7 +30,15 @@ namespace msx::hk {
 // with the zero padding vanish). SUMS: 1, the row sums of op(A) over K; 2, the column sums of
 // op(B) (a bias gradient), taken from the fragments of the waves of the first wave column (row).
 
-template <int BM, int BN, int WGM, int WGN, int BK, bool AKC, bool BKC, int NS, bool FP, int SUMS>
+//
+// ROWS: the same products with the operands exchanged, C tiles: a lane holds four rows of one output
+// column, and 16 lanes store 64 consecutive bytes of a row. For outputs whose rows are not 16-byte
+// aligned (a prediction of 30522 classes, packed): a lane's four columns there are four 4-byte
+// stores, each instruction touching 64 separate pieces of 16 rows. 4096 x 30522 x 128: 459 us by
+// columns, 385 by rows (the products take 206 at the MFMA rate, leaving the stores out 344); by rows
+// tiles of 128 x 64 408, 128 x 128 396 to 470, K tiles of 32 408, four stages 434, streaming stores
+// or rows of tiles first the same.
+template <int BM, int BN, int WGM, int WGN, int BK, bool AKC, bool BKC, int NS, bool FP, int SUMS, bool ROWS = false>
 __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_lds(GemmPtrs ptrs, int64_t M, int64_t N, int64_t K,
                                                              int64_t lda, int64_t ldb, int64_t ldc, int64_t kchunk,
                                                              int64_t zero_to, bool vo, GemmOrder order) {
@@ -141,9 +149,14 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_lds(GemmPtrs ptrs, int6
   for (int j = 0; j < J; ++j) {
     bias4[j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     if (bias && !ws) {
-      const int64_t col0 = n0 + wn + (BKC ? 16 * j + 4 * q : 4 * J * q + 4 * j);
+      if constexpr (ROWS) {
+        const int64_t col = n0 + wn + (BKC ? 16 * j + c : J * c + j);
+        bias4[j][0] = col < N ? bias[col] : 0.0f;
+      } else {
+        const int64_t col0 = n0 + wn + (BKC ? 16 * j + 4 * q : 4 * J * q + 4 * j);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) bias4[j][u] = col0 + u < N ? bias[col0 + u] : 0.0f;
+        for (int u = 0; u < 4; ++u) bias4[j][u] = col0 + u < N ? bias[col0 + u] : 0.0f;
+      }
     }
   }
   v4f acc[I][J];
@@ -207,7 +220,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_lds(GemmPtrs ptrs, int6
           for (int j = 0; j < J; ++j) {
             const float a = AKC ? f.a[kb][i][s] : f.a[kb][s][i];
             const float b = BKC ? f.b[kb][j][s] : f.b[kb][s][j];
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b, a, acc[i][j], 0, 0, 0);
+            acc[i][j] = ROWS ? __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc[i][j], 0, 0, 0)
+                             : __builtin_amdgcn_mfma_f32_16x16x4f32(b, a, acc[i][j], 0, 0, 0);
           }
       if (SUMS != 0 && sum_wave) {
 #pragma unroll
@@ -256,42 +270,62 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_lds(GemmPtrs ptrs, int6
   wait_vm(0);  // no load may still write LDS when the block ends
   float* out = ws ? ws + int64_t(tz) * M * N : ptrs.c[0];
   const int64_t ldo = ws ? N : ldc, zto = ws ? N : zero_to;
+  if constexpr (ROWS) {
+    const bool more = !ws && (epi.act != EPI_NONE || epi.addend || epi.drop_token);
+    const GemmEpi rest{nullptr, epi.addend, epi.pre_in, epi.pre_out, epi.act, epi.drop_token, epi.drop_threshold,
+                       epi.drop_scale, epi.drop_seed, epi.pre16};
 #pragma unroll
-  for (int i = 0; i < I; ++i) {
-    const int64_t row = m0 + wm + (AKC ? 16 * i + c : I * c + i);
-    if (row >= M) continue;
-    float* orow = out + row * ldo;
+    for (int i = 0; i < I; ++i)
 #pragma unroll
-    for (int j = 0; j < J; ++j) {
-      int64_t col;
-      v4f v;
-      if (BKC) {
-        col = n0 + wn + 16 * j + 4 * q;
-        v = acc[i][j] + bias4[j];
-      } else {
-        // Columns wn + J (4 q + r) + jj: group j holds r = (4 j + u) / J, jj = (4 j + u) % J.
-        col = n0 + wn + 4 * J * q + 4 * j;
+      for (int u = 0; u < 4; ++u) {
+        const int64_t row = m0 + wm + (AKC ? 16 * i + 4 * q + u : I * (4 * q + u) + i);
+        if (row >= M) continue;
+        float* orow = out + row * ldo;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = acc[i][(4 * j + u) % J][(4 * j + u) / J];
-        v += bias4[j];
-      }
-      // The rest of the epilogue (activation or its gradient, addend, dropout gradient) after the
-      // bias, as the other kernel applies it.
-      const bool more = !ws && (epi.act != EPI_NONE || epi.addend || epi.drop_token);
-      if (vo && col + 3 < N) {
-        if (more) {
-          const float4 f = gemm_epilogue4(GemmEpi{nullptr, epi.addend, epi.pre_in, epi.pre_out, epi.act, epi.drop_token,
-                                                  epi.drop_threshold, epi.drop_scale, epi.drop_seed, epi.pre16},
-                                          make_float4(v[0], v[1], v[2], v[3]), row, col, ldo);
-          v = v4f{f.x, f.y, f.z, f.w};
+        for (int j = 0; j < J; ++j) {
+          const int64_t col = n0 + wn + (BKC ? 16 * j + c : J * c + j);
+          const float v = acc[i][j][u] + bias4[j][0];
+          if (col < zto) orow[col] = col < N ? (more ? gemm_epilogue(rest, v, row, col, ldo) : v) : 0.0f;
         }
-        *reinterpret_cast<v4f*>(orow + col) = v;
-      } else {
-        const GemmEpi rest{nullptr, epi.addend, epi.pre_in, epi.pre_out, epi.act, epi.drop_token, epi.drop_threshold,
-                           epi.drop_scale, epi.drop_seed, epi.pre16};
+      }
+  } else {
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-          if (col + u < zto) orow[col + u] = col + u < N ? (more ? gemm_epilogue(rest, v[u], row, col + u, ldo) : v[u]) : 0.0f;
+    for (int i = 0; i < I; ++i) {
+      const int64_t row = m0 + wm + (AKC ? 16 * i + c : I * c + i);
+      if (row >= M) continue;
+      float* orow = out + row * ldo;
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        int64_t col;
+        v4f v;
+        if (BKC) {
+          col = n0 + wn + 16 * j + 4 * q;
+          v = acc[i][j] + bias4[j];
+        } else {
+          // Columns wn + J (4 q + r) + jj: group j holds r = (4 j + u) / J, jj = (4 j + u) % J.
+          col = n0 + wn + 4 * J * q + 4 * j;
+#pragma unroll
+          for (int u = 0; u < 4; ++u) v[u] = acc[i][(4 * j + u) % J][(4 * j + u) / J];
+          v += bias4[j];
+        }
+        // The rest of the epilogue (activation or its gradient, addend, dropout gradient) after the
+        // bias, as the other kernel applies it.
+        const bool more = !ws && (epi.act != EPI_NONE || epi.addend || epi.drop_token);
+        if (vo && col + 3 < N) {
+          if (more) {
+            const float4 f = gemm_epilogue4(GemmEpi{nullptr, epi.addend, epi.pre_in, epi.pre_out, epi.act, epi.drop_token,
+                                                    epi.drop_threshold, epi.drop_scale, epi.drop_seed, epi.pre16},
+                                            make_float4(v[0], v[1], v[2], v[3]), row, col, ldo);
+            v = v4f{f.x, f.y, f.z, f.w};
+          }
+          *reinterpret_cast<v4f*>(orow + col) = v;
+        } else {
+          const GemmEpi rest{nullptr, epi.addend, epi.pre_in, epi.pre_out, epi.act, epi.drop_token, epi.drop_threshold,
+                             epi.drop_scale, epi.drop_seed, epi.pre16};
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (col + u < zto) orow[col + u] = col + u < N ? (more ? gemm_epilogue(rest, v[u], row, col + u, ldo) : v[u]) : 0.0f;
+        }
       }
     }
   }
@@ -370,14 +404,16 @@ bool gemm_lds(hipStream_t s, const GemmArgs& g, const GemmPtrs& ptrs, int split,
                         : (g.ldc % 4 == 0 && a16(g.c) && a16(g.addend) && a16(g.pre_in) && a16(g.pre_out));
     const int64_t zero_to = g.pad_c ? g.ldc : g.n;
     const int sums = g.colsum ? (g.sum_a ? 1 : 2) : 0;
-#define MSX_LDS(BM, BN, WGM, WGN, BK, AK, BKC_, NS, FP, S)                                                         \
-  MSX_LAUNCH((k_gemm_lds<BM, BN, WGM, WGN, BK, AK, BKC_, NS, FP, S>), lgrid, dim3(64 * WGM * WGN), 0, s, ptrs, g.m, \
-             g.n, g.k, g.lda, g.ldb, g.ldc, chunk, zero_to, lvo, lorder)
+#define MSX_LDS(BM, BN, WGM, WGN, BK, AK, BKC_, NS, FP, S, ...)                                                    \
+  MSX_LAUNCH((k_gemm_lds<BM, BN, WGM, WGN, BK, AK, BKC_, NS, FP, S __VA_OPT__(,) __VA_ARGS__>), lgrid,              \
+             dim3(64 * WGM * WGN), 0, s, ptrs, g.m, g.n, g.k, g.lda, g.ldb, g.ldc, chunk, zero_to, lvo, lorder)
 #define MSX_LDS_S(BM, BN, WGM, WGN, BK, AK, BKC_, NS, FP)          \
   if (sums == 1) MSX_LDS(BM, BN, WGM, WGN, BK, AK, BKC_, NS, FP, 1); \
   else if (sums == 2) MSX_LDS(BM, BN, WGM, WGN, BK, AK, BKC_, NS, FP, 2); \
   else MSX_LDS(BM, BN, WGM, WGN, BK, AK, BKC_, NS, FP, 0)
-    if (akc && bkc) { MSX_LDS_S(64, 64, 2, 2, 16, true, true, 3, true); }
+    // Unaligned output rows (and no sums, which only padded gradients carry): by rows.
+    if (akc && bkc && !lvo && sums == 0) { MSX_LDS(64, 64, 2, 2, 16, true, true, 3, true, 0, true); }
+    else if (akc && bkc) { MSX_LDS_S(64, 64, 2, 2, 16, true, true, 3, true); }
     else if (akc) { MSX_LDS_S(64, 128, 2, 4, 32, true, false, 3, true); }
     else if (!bkc) { MSX_LDS_S(128, 128, 2, 2, 32, false, false, 3, false); }
     else { MSX_LDS_S(64, 64, 2, 2, 16, false, true, 3, true); }

@@ -56,6 +56,9 @@ struct Launch {
   // A launch whose outputs are none of its inputs (a GEMM, attention): running it again recomputes
   // the same values, so a profile may time it over back-to-back repeats.
   bool pure = false;
+  // A launch of the forward program that only forms its loss, which a held-out evaluation, reducing
+  // the prediction itself, does not read.
+  bool loss_only = false;
 };
 
 struct RunStats {
@@ -227,7 +230,7 @@ class Executor {
   // Packs `batch` (and checks ids, labels and key masks) into the next pinned slot and enqueues
   // its copy to the device input block.
   void stage(const BatchView& batch);
-  void run(hipStream_t s);  // every launch, in order
+  void run(hipStream_t s, bool with_loss = true);  // every launch, in order (but the loss_only ones)
   const std::vector<Launch>& launches() const { return launches_; }
   // The launch plan as text: one line a launch (its place, the values it completes, side stream,
   // algorithmic flop and bytes), then the buffer plan (every value's arena slice).

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 from ops_lib import Prog, fast_values, within
+from test_gpu_heldout import batches_of, load_logits
 from test_gpu_ops import both
 
 pytestmark = pytest.mark.gpu
@@ -149,3 +150,56 @@ def test_mixed_chains_of_products(mixed, rows, h):
     for a, w in ((a1, w1), (a2, w2), (a3, w3)):
         want, mag = want + f16(a) @ f16(w).T, mag + np.abs(f16(a)) @ np.abs(f16(w)).T
     assert np.max(np.abs(got - want) / mag) <= 1e-5
+
+
+@pytest.mark.parametrize("m,k,n,bias", [(70, 48, 30522, True), (4099, 32, 515, False), (37, 144, 60001, True), (2100, 16, 1001, False)])
+def test_gemm_of_unaligned_output_rows(ctx, m, k, n, bias):
+    """x wᵀ (+ b) into rows that are not 16-byte aligned, against float64 (1e-6 of the sum of |terms|
+    and the bias: f32 accumulation of up to 144 terms)."""
+    rng = np.random.default_rng(n)
+    x, wt = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32)
+    b = rng.standard_normal(n).astype(np.float32)
+    p = Prog()
+    y = p.op("MatMul", [p.input("x", x.shape), p.op("Transpose", [p.input("w", wt.shape)], (k, n))], (m, n))
+    if bias:
+        y = p.op("AddRows", [y, p.input("b", b.shape)], (m, n))
+    p.out(y)
+    prog = ctx.program(p.text())
+    prog.run({"x": x, "w": wt, **({"b": b} if bias else {})})
+    got = prog.output(0, m * n).reshape(m, n)
+    X, W, bb = x.astype(np.float64), wt.astype(np.float64), b.astype(np.float64) * bias
+    worst = np.max(np.abs(got - (X @ W.T + bb)) / (1e-6 * (np.abs(X) @ np.abs(W).T + np.abs(bb)) + 1e-30))
+    assert worst <= 1.0, worst
+
+
+@pytest.mark.parametrize("v", [8192, 8193, 16384, 16385, 32768, 32769])
+def test_held_out_rows_of_many_classes(ctx, oracle, v):
+    """The held-out reduction at the edges of its register-resident rows: ties across waves, a NaN, an
+    infinity, -inf logits and a row of nothing else."""
+    rows = 9
+    rng = np.random.default_rng(v)
+    x = (rng.standard_normal((1, rows, v)) * 4).astype(np.float32)
+    labels = rng.integers(0, v, (1, rows)).astype(np.int32)
+    weights = np.ones((1, rows), np.float32)
+    x[0, 0, [5, 1029, v - 1]] = 40.0
+    labels[0, 0] = 5
+    x[0, 1, [v - 2, v - 1]] = 40.0
+    labels[0, 1] = v - 2
+    x[0, 2, 7:v - 3] = -np.inf
+    labels[0, 2] = int(np.argmax(x[0, 2]))
+    load_logits(ctx, rows, v)
+    for case in ("finite", "nan", "inf", "all -inf"):
+        if case == "nan":
+            x[0, 3, v - 1] = np.nan
+        elif case == "inf":
+            x[0, 3, v - 1] = np.inf
+        elif case == "all -inf":
+            x[0, 4, :] = -np.inf
+            labels[0, 4] = 0
+        got = ctx.evaluate(batches_of(x, labels, weights), "labels", "weights")
+        want = oracle.held_out_tally(x, labels, weights)
+        assert got["correct"] == want["correct"] and got["selected"] == want["selected"], case
+        if case == "finite":
+            assert abs(got["loss"] - want["loss"]) <= 1e-5 * abs(want["loss"]) + 1e-6
+        else:
+            assert np.isnan(got["loss"]) == np.isnan(want["loss"]), case
