@@ -26,6 +26,14 @@ void elementwise(hipStream_t s, int op, const float* a, const float* b, float* o
 void elementwise2(hipStream_t s, int op1, const float* a, const float* b, int op2, const float* sc, bool inner_left,
                   float* o, int64_t n);
 void fill_from(hipStream_t s, const float* scalar, float* o, int64_t n);  // BroadcastScalar
+// A step's host inputs from the ring of pinned slots: `words` 8-byte words of slot state[0] % 4 to
+// `dst`; then state[0] + 1, which is also written to the host word `done`. state[1] is the kernel's.
+struct FetchRing {
+  const void* base;  // 4 slots of slot_bytes
+  size_t slot_bytes;
+};
+constexpr uint32_t kFetchSlots = 4;
+void fetch_inputs(hipStream_t s, const FetchRing& ring, void* dst, int64_t words, uint32_t* state, uint32_t* done);
 void fill_zero(hipStream_t s, void* o, int64_t bytes);                     // kernel, not a memset
 // y[r, c] = f16(x[r, c]) (round to nearest even) for r < rows, c < cols; rows ldx / ldy apart.
 void to_f16_rows(hipStream_t s, const float* x, int64_t ldx, _Float16* y, int64_t ldy, int64_t rows, int64_t cols);

@@ -98,6 +98,42 @@ void fill_zero(hipStream_t s, void* o, int64_t bytes) {
                      static_cast<uint32_t*>(o), words);
 }
 
+// The host inputs of a step, copied by the step itself: as the first kernel of its graph it costs one
+// dispatch, where a copy command between two graphs idles the device for a submission, a copy and
+// two waits (a step of the linear regression: 28.3 us with the copy command, 24.3 here; of the MLP of
+// 784 inputs, 200 KB a step, 95.3 and 68.7). Which slot is in device memory, so that one captured graph serves all. The
+// loads are of system scope (the slots are host memory, rewritten between steps), 8 bytes each, four
+// in flight a thread. The last block to finish moves the slot on: by then every block has read it.
+__global__ __launch_bounds__(256) void k_fetch_inputs(FetchRing ring, unsigned long long* __restrict__ dst, int64_t words,
+                                                      uint32_t* __restrict__ state, uint32_t* __restrict__ done) {
+  const uint32_t step = __hip_atomic_load(state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const unsigned long long* src = reinterpret_cast<const unsigned long long*>(
+      static_cast<const char*>(ring.base) + size_t(step % kFetchSlots) * ring.slot_bytes);
+  const int64_t at = int64_t(blockIdx.x) * 1024 + threadIdx.x;
+  unsigned long long t[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+    if (at + 256 * u < words) t[u] = __hip_atomic_load(src + at + 256 * u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+    if (at + 256 * u < words) dst[at + 256 * u] = t[u];
+  __syncthreads();
+  if (threadIdx.x == 0 &&
+      __hip_atomic_fetch_add(state + 1, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
+    __hip_atomic_store(state + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(state, step + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(done, step + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+void fetch_inputs(hipStream_t s, const FetchRing& ring, void* dst, int64_t words, uint32_t* state, uint32_t* done) {
+  if (words <= 0) return;
+  if (reinterpret_cast<uintptr_t>(ring.base) % 8 || reinterpret_cast<uintptr_t>(dst) % 8 || ring.slot_bytes % 8 ||
+      size_t(words) * 8 > ring.slot_bytes)
+    bad("fetch_inputs needs whole 8-byte words inside a slot");
+  MSX_LAUNCH(k_fetch_inputs, dim3(blocks_for(words, 1024)), dim3(256), 0, s, ring, static_cast<unsigned long long*>(dst),
+             words, state, done);
+}
+
 __global__ __launch_bounds__(256) void k_to_f16_rows(const float* __restrict__ x, int64_t ldx, _Float16* __restrict__ y,
                                                      int64_t ldy, int64_t rows, int64_t cols) {
   const int64_t n = rows * cols;

@@ -2,6 +2,8 @@
 #include "runtime.h"
 
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -11,6 +13,7 @@
 #include <memory>
 #include <mutex>
 #include <set>
+#include <thread>
 
 // The device memory of Session::held_out_static: the row results [rows, 2] of at most
 // kStaticEvalRows rows, then the HeldOutState at the next 256-byte boundary (512 KiB + 256 bytes).
@@ -99,17 +102,17 @@ Resolved resolve(const Program& p, uint32_t v) {
 Executor::Executor(Session& s, const Program& p, bool is_step) : s_(s), p_(p), is_step_(is_step) {
   build();
   if (s_.opt_.plan_only) return;
-  for (int i = 0; i < kRing; ++i) {
-    hip_check(hipHostMalloc(&pinned_[i], std::max<size_t>(input_bytes_, 256), hipHostMallocDefault), "hipHostMalloc");
-    hip_check(hipEventCreateWithFlags(&slot_done_[i], hipEventDisableTiming), "hipEventCreate");
-  }
+  slot_bytes_ = std::max<size_t>(host_bytes_, 256);
+  void* mem = nullptr;
+  hip_check(hipHostMalloc(&mem, hk::kFetchSlots * slot_bytes_ + 256, hipHostMallocMapped | hipHostMallocCoherent),
+            "hipHostMalloc");
+  pinned_ = static_cast<char*>(mem);
+  *fetched() = 0;
+  fetch_state_ = s_.fetch_state_ + (is_step_ ? 0 : 32);
 }
 
 Executor::~Executor() {
-  for (int i = 0; i < kRing; ++i) {
-    if (slot_done_[i]) (void)hipEventDestroy(slot_done_[i]);
-    if (pinned_[i]) (void)hipHostFree(pinned_[i]);
-  }
+  if (pinned_) (void)hipHostFree(pinned_);
 }
 
 void* Executor::ptr(uint32_t id) const {
@@ -2323,10 +2326,25 @@ void Executor::stage(const BatchView& batch) {
       if (!any) throw IrError("key mask `" + name + "`: sequence " + std::to_string(b) + " has no unmasked key");
     }
   }
-  int slot = next_slot_;
-  next_slot_ = (next_slot_ + 1) % kRing;
-  hip_check(hipEventSynchronize(slot_done_[slot]), "hipEventSynchronize (staging slot)");
-  char* host = static_cast<char*>(pinned_[slot]);
+  // The slot was last read by the fetch kFetchSlots fetches ago. Polled: a step is mostly waited out
+  // within the time of a call into the driver; a long one is looked at every 50 us.
+  const volatile uint32_t* done = fetched();
+  auto landed = [&] { return int32_t(*done + hk::kFetchSlots - fetches_) > 0; };
+  if (host_bytes_ && !landed()) {
+    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+    while (!landed() && std::chrono::steady_clock::now() < until) std::this_thread::yield();
+    while (!landed()) {
+      const hipError_t e = hipStreamQuery(s_.stream_);
+      if (e != hipErrorNotReady) {
+        hip_check(e, "staging slot");
+        if (landed()) break;
+        throw HipError("a staging slot is still in use and its stream is idle");
+      }
+      std::this_thread::sleep_for(std::chrono::microseconds(50));
+    }
+  }
+  std::atomic_thread_fence(std::memory_order_acquire);
+  char* host = pinned_ + size_t(fetches_ % hk::kFetchSlots) * slot_bytes_;
   if (s_.corpus_) {
     auto it = batch.i32.find(kDrawInput);
     if (it == batch.i32.end() || it->second.size() != 3 + s_.corpus_batch_)
@@ -2354,14 +2372,18 @@ void Executor::stage(const BatchView& batch) {
     if (it == batch.i32.end() || int64_t(it->second.size()) != ps.n) throw IrError("missing input `" + ps.ids_name + "`");
     hk::eg_plan_host(it->second.data(), ps.n, ps.rows, reinterpret_cast<int32_t*>(host + ps.offset));
   }
-  if (host_bytes_) {
-    hip_check(hipMemcpyAsync(arena_.at(input_token_), host, host_bytes_, hipMemcpyHostToDevice, s_.stream_), "hipMemcpyAsync (inputs)");
-    s_.stats_.bytes_uploaded += host_bytes_;
-  }
-  hip_check(hipEventRecord(slot_done_[slot], s_.stream_), "hipEventRecord");
+  s_.stats_.bytes_uploaded += host_bytes_;
 }
 
-void Executor::run(hipStream_t s, bool with_loss) {
+void Executor::fetch(hipStream_t s, bool captured) {
+  if (!host_bytes_) return;
+  hk::fetch_inputs(s, {pinned_, slot_bytes_}, arena_.at(input_token_), int64_t(host_bytes_ / 8), fetch_state_, fetched());
+  hip_check(hipGetLastError(), "input fetch");
+  if (!captured) replayed();
+}
+
+void Executor::run(hipStream_t s, bool with_loss, bool captured) {
+  fetch(s, captured);
   // Side launches are held and issued on the side stream eight at a time, forked from the main
   // stream's work so far; the main stream joins them at the first launch after the backward and
   // at the end (under capture these are graph edges, not nodes). Each fork and join is a wait
@@ -2497,7 +2519,7 @@ Session::Session(int device, const TrainingStep& step, const Program& forward, u
     if (pass == 0) trained_ = at;
   }
   total_ = std::max<int64_t>(at, 64);
-  size_t floats = size_t(total_) * 4 + loss_capacity_ + 64;
+  size_t floats = size_t(total_) * 4 + loss_capacity_ + 128;
   hip_check(hipMalloc(&state_mem_, floats * 4), "hipMalloc (parameter state)");
   hip_check(hipMemset(state_mem_, 0, floats * 4), "hipMemset (parameter state)");
   float* base = static_cast<float*>(state_mem_);
@@ -2507,6 +2529,7 @@ Session::Session(int device, const TrainingStep& step, const Program& forward, u
   v_ = base + 3 * total_;
   losses_dev_ = base + 4 * total_;
   counter_ = reinterpret_cast<uint32_t*>(base + 4 * total_ + loss_capacity_);
+  fetch_state_ = counter_ + 64;
   if (opt_.mixed) {
     hip_check(hipMalloc(&param16_, size_t(total_) * 2), "hipMalloc (f16 parameters)");
     hip_check(hipMemset(param16_, 0, size_t(total_) * 2), "hipMemset (f16 parameters)");
@@ -2638,7 +2661,7 @@ void Session::run_step(const BatchView& batch) {
     if (!graph_exec_) {
       hip_check(hipStreamBeginCapture(stream_, hipStreamCaptureModeRelaxed), "hipStreamBeginCapture");
       try {
-        step_exec_->run(stream_);
+        step_exec_->run(stream_, true, true);
       } catch (...) {
         hipGraph_t g = nullptr;
         (void)hipStreamEndCapture(stream_, &g);
@@ -2652,6 +2675,7 @@ void Session::run_step(const BatchView& batch) {
       stats_.kernels_per_step = nodes;
     }
     hip_check(hipGraphLaunch(graph_exec_, stream_), "hipGraphLaunch");
+    step_exec_->replayed();
     stats_.graph_launches += 1;
   } else {
     step_exec_->run(stream_);
@@ -2666,6 +2690,7 @@ void Session::run_step(const BatchView& batch) {
 std::vector<Session::Timed> Session::profile_step(const StepInputs& in) {
   constexpr int kRepeats = 10;
   step_exec_->stage(in.batch);
+  step_exec_->fetch(stream_, false);
   const auto& ls = step_exec_->launches();
   std::vector<hipEvent_t> ev(4 * ls.size());
   for (auto& e : ev) hip_check(hipEventCreate(&e), "hipEventCreate");

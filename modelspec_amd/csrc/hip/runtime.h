@@ -194,6 +194,7 @@ class Session : public Engine {
   // every upload and every optimizer step.
   _Float16* param16_ = nullptr;
   float* losses_dev_ = nullptr;
+  uint32_t* fetch_state_ = nullptr;  // two words for each executor
   uint32_t* counter_ = nullptr;
   uint32_t loss_capacity_ = 1u << 20;
   void* state_mem_ = nullptr;
@@ -227,10 +228,15 @@ class Executor {
  public:
   Executor(Session& s, const Program& p, bool is_step);
   ~Executor();
-  // Packs `batch` (and checks ids, labels and key masks) into the next pinned slot and enqueues
-  // its copy to the device input block.
+  // Packs `batch` (and checks ids, labels and key masks) into the pinned slot that the next run
+  // copies to the device input block.
   void stage(const BatchView& batch);
-  void run(hipStream_t s, bool with_loss = true);  // every launch, in order (but the loss_only ones)
+  // The copy of the staged slot: the first launch of a run. A captured one is counted by replayed()
+  // each time its graph is launched.
+  void fetch(hipStream_t s, bool captured);
+  void replayed() { fetches_ += host_bytes_ ? 1 : 0; }
+  // Every launch, in order (but the loss_only ones).
+  void run(hipStream_t s, bool with_loss = true, bool captured = false);
   const std::vector<Launch>& launches() const { return launches_; }
   // The launch plan as text: one line a launch (its place, the values it completes, side stream,
   // algorithmic flop and bytes), then the buffer plan (every value's arena slice).
@@ -260,10 +266,12 @@ class Executor {
   std::vector<PlanSlot> plan_slots_;
   size_t input_bytes_ = 0, host_bytes_ = 0, draw_offset_ = 0;
   void* input_token_ = nullptr;
-  static constexpr int kRing = 4;
-  void* pinned_[kRing] = {};
-  hipEvent_t slot_done_[kRing] = {};
-  int next_slot_ = 0;
+  // hk::kFetchSlots pinned slots of slot_bytes_, then the word in which the device counts its fetches.
+  char* pinned_ = nullptr;
+  size_t slot_bytes_ = 0;
+  uint32_t* fetch_state_ = nullptr;  // device: the fetch kernel's
+  uint32_t fetches_ = 0;             // fetches launched; the next staged slot is fetches_ % kFetchSlots
+  uint32_t* fetched() const { return reinterpret_cast<uint32_t*>(pinned_ + hk::kFetchSlots * slot_bytes_); }
   // id checks before upload: input name -> rows it indexes (Embedding / EmbeddingGrad / labels)
   std::map<std::string, int64_t> id_bounds_;
   std::vector<std::string> key_masks_;

@@ -3,6 +3,7 @@ largest of a dispatch's range), against the oracle under the reference's per-ker
 import numpy as np
 import pytest
 
+from modelspec_amd import api
 from ops_lib import Prog, fast_values, within
 from test_gpu_heldout import batches_of, load_logits
 from test_gpu_ops import both
@@ -203,3 +204,32 @@ def test_held_out_rows_of_many_classes(ctx, oracle, v):
             assert abs(got["loss"] - want["loss"]) <= 1e-5 * abs(want["loss"]) + 1e-6
         else:
             assert np.isnan(got["loss"]) == np.isnan(want["loss"]), case
+
+
+def test_each_step_reads_its_own_inputs(ctx):
+    """Eleven steps through the four staging slots, in one call, one by one, and one by one with a
+    refused call before each (it uses no slot): the same losses, all different."""
+    step, fwd = api.compile_config("mlp_micro")
+    rng = np.random.default_rng(3)
+    shapes = ((784, 256), (256,), (256, 10), (10,))
+    values = [rng.standard_normal(s).astype(np.float32) * 0.05 for s in shapes]
+    batches = [{"x": rng.random((8, 784), np.float32), "labels": rng.integers(0, 10, 8).astype(np.int32),
+                "weights": np.ones(8, np.float32)} for _ in range(11)]
+    ctx.load(step, fwd, 0, 1)
+    got = []
+    for how in ("one call", "one by one", "after refusals"):
+        ctx.set_params(values)
+        if how == "one call":
+            got.append(ctx.run_steps(batches))
+            continue
+        losses = []
+        for b in batches:
+            if how == "after refusals":
+                with pytest.raises(api.MsxError):
+                    ctx.run_steps([{k: v for k, v in b.items() if k != "weights"}])
+                with pytest.raises(api.MsxError):
+                    ctx.run_steps([dict(b, labels=b["labels"] + 10)])
+            losses.append(ctx.run_steps([b])[0])
+        got.append(np.array(losses))
+    assert len(set(got[0].tolist())) == 11
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
