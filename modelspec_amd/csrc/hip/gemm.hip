@@ -61,7 +61,7 @@ namespace {
 // V: the group is 16-byte aligned and wholly in or out of range, or its out-of-range part lies in
 // zero padding of the rows: one float4 load; otherwise four clamped scalar loads.
 // The cross-entropy gradient of logit x at column c of a row with entry t = (max, 1 / sum,
-// g w / sum(w), label): (g w / sum(w)) (exp(x - max) / sum - [c = label]), in k_ce_rows' operation
+// g w / sum(w), label): (g w / sum(w)) (exp(x - max) / sum - [c = label]), in k_ce_rows_p's operation
 // order; 0 past the row's `cols` columns and in a row of a batch whose weights sum to 0.
 __device__ __forceinline__ float ce_grad_of(float x, const float4 t, int64_t c, int64_t cols) {
   const int lab = __float_as_int(t.w);
@@ -78,7 +78,6 @@ __device__ __forceinline__ float4 wide_load(const float* __restrict__ P, int64_t
   if (KC) { r = e / (WK / 4); k = (e % (WK / 4)) * 4; } else { k = e / (R / 4); r = (e % (R / 4)) * 4; }
   const int64_t gr = r0 + r, gk = k0 + k;
   if (V) {
-    const bool ok = gr < rows && gk < kend;
     // A group past the end reads the aligned group holding the last element instead.
     const int64_t cr = KC ? (gr < rows ? gr : rows - 1) : (gr < rows ? gr : (rows - 1) & ~int64_t(3));
     const int64_t ck = KC ? (gk < kend ? gk : (kend - 1) & ~int64_t(3)) : (gk < kend ? gk : kend - 1);
@@ -89,7 +88,7 @@ __device__ __forceinline__ float4 wide_load(const float* __restrict__ P, int64_t
       f = make_float4(ce_grad_of(f.x, t, scol, cols), ce_grad_of(f.y, t, scol + 1, cols),
                       ce_grad_of(f.z, t, scol + 2, cols), ce_grad_of(f.w, t, scol + 3, cols));
     }
-    return ok ? f : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    return f;
   }
   float v[4];
 #pragma unroll
@@ -98,9 +97,18 @@ __device__ __forceinline__ float4 wide_load(const float* __restrict__ P, int64_t
     const int64_t cr = rr < rows ? rr : rows - 1, ck = kk < kend ? kk : kend - 1;
     float x = KC ? P[cr * ld + ck] : P[ck * ld + cr];
     if (XF) x = ce_grad_of(x, tab[KC ? cr : ck], KC ? ck : cr, cols);
-    v[j] = rr < rows && kk < kend ? x : 0.0f;
+    v[j] = x;
   }
   return make_float4(v[0], v[1], v[2], v[3]);
+}
+// wide_load's group with its elements past kend zeroed: applied where the group is stored to LDS, so
+// that nothing waits for a load before its tile is due, and to the last K tile only. (A row past the
+// end holds a copy of the last one: its products go to outputs that are not stored.)
+template <bool KC, int R, int WK, bool V>
+__device__ __forceinline__ float4 wide_mask(float4 f, int64_t kend, int64_t k0, int e) {
+  const int64_t gk = k0 + (KC ? (e % (WK / 4)) * 4 : e / (R / 4));
+  auto in = [&](int j) { return KC && !V ? gk + j < kend : gk < kend; };
+  return make_float4(in(0) ? f.x : 0.0f, in(1) ? f.y : 0.0f, in(2) ? f.z : 0.0f, in(3) ? f.w : 0.0f);
 }
 // The column a KC operand's element (row r, k) takes in its [k][row] LDS tile: r XOR a multiple of
 // 128 / WK chosen by k / 4. A float4 group's four stores (k .. k + 3 of one row) go to four rows of
@@ -255,13 +263,24 @@ __global__ __launch_bounds__(256) void k_gemm_w(GemmPtrs ptrs, int64_t M, int64_
     else
       return wide_load<TB, TN, WK, VB, CE == 2>(B, ldb, N, kend, n0, k0, gb(h), ce_tab, ptrs.ce_cols);
   };
-  float4 ra[HA], rb[HB];
+  // The next PF K tiles are in flight in registers (a group of each operand a thread and tile): a
+  // launch of few blocks waits for memory, not for the MFMAs, with one tile ahead (64 x 256 x 784,
+  // 16 blocks: 13.9 us with one, 10.9 with four and the fragments below read together). The same
+  // products in the same order.
+  constexpr int PF = !H && CE == 0 && NB == 2 && HA + HB <= 2 ? 4 : 1;
+  float4 ra[PF][HA], rb[PF][HB];
+  auto fetch = [&](int64_t k0, float4 (&xa)[HA], float4 (&xb)[HB]) {
+    if constexpr (KS) advance(k0);
 #pragma unroll
-  for (int h = 0; h < HA; ++h)
-    if (GA % 256 == 0 || tid + 256 * h < GA) ra[h] = load_a(kbeg, h);
+    for (int h = 0; h < HA; ++h)
+      if (GA % 256 == 0 || tid + 256 * h < GA) xa[h] = load_a(k0, h);
 #pragma unroll
-  for (int h = 0; h < HB; ++h)
-    if (GB % 256 == 0 || tid + 256 * h < GB) rb[h] = load_b(kbeg, h);
+    for (int h = 0; h < HB; ++h)
+      if (GB % 256 == 0 || tid + 256 * h < GB) xb[h] = load_b(k0, h);
+  };
+#pragma unroll
+  for (int u = 0; u < PF; ++u)
+    if (u == 0 || kbeg + u * WK < kend) fetch(kbeg + u * WK, ra[u], rb[u]);
   // Column sums: thread t adds tile column t mod T over the K rows (t / T) per .. + per of each
   // K tile, per = WK / (256 / T).
   const int T = sum_a ? TM : TN;
@@ -271,42 +290,40 @@ __global__ __launch_bounds__(256) void k_gemm_w(GemmPtrs ptrs, int64_t M, int64_
   const bool sum_kc = sum_a ? !TA : TB;
   const int sum_k0 = (tid / T) * sum_per, sum_col = tid % T;
   float csum = 0.0f;
-  int buf = 0;
-  for (int64_t k0 = kbeg; k0 < kend; k0 += WK) {
+  // K tile k0, its groups in xa and xb; `more`: tile k0 + PF WK exists.
+  auto tile = [&](int64_t k0, int buf, float4 (&xa)[HA], float4 (&xb)[HB], bool more) {
     if (NB == 1 && k0 != kbeg) __syncthreads();  // the single buffer is free again
+    if (k0 + WK > kend) {
+#pragma unroll
+      for (int h = 0; h < HA; ++h) xa[h] = wide_mask<!TA, TM, WK, VA>(xa[h], kend, k0, ga(h));
+#pragma unroll
+      for (int h = 0; h < HB; ++h) xb[h] = wide_mask<TB, TN, WK, VB>(xb[h], kend, k0, gb(h));
+    }
     if constexpr (H) {
       if constexpr (RA) {
-        rows_store_h<TM, PH, HA>(Ah0 + buf * (TM * PH), tid, ra);
+        rows_store_h<TM, PH, HA>(Ah0 + buf * (TM * PH), tid, xa);
       } else {
 #pragma unroll
         for (int h = 0; h < HA; ++h)
-          if (GA % 256 == 0 || tid + 256 * h < GA) wide_store_h<!TA, TM, PH, WK>(Ah0 + buf * (TM * PH), tid + 256 * h, ra[h]);
+          if (GA % 256 == 0 || tid + 256 * h < GA) wide_store_h<!TA, TM, PH, WK>(Ah0 + buf * (TM * PH), tid + 256 * h, xa[h]);
       }
       if constexpr (RB) {
-        rows_store_h<TN, PH, HB>(Bh0 + buf * (TN * PH), tid, rb);
+        rows_store_h<TN, PH, HB>(Bh0 + buf * (TN * PH), tid, xb);
       } else {
 #pragma unroll
         for (int h = 0; h < HB; ++h)
-          if (GB % 256 == 0 || tid + 256 * h < GB) wide_store_h<TB, TN, PH, WK>(Bh0 + buf * (TN * PH), tid + 256 * h, rb[h]);
+          if (GB % 256 == 0 || tid + 256 * h < GB) wide_store_h<TB, TN, PH, WK>(Bh0 + buf * (TN * PH), tid + 256 * h, xb[h]);
       }
     } else {
 #pragma unroll
       for (int h = 0; h < HA; ++h)
-        if (GA % 256 == 0 || tid + 256 * h < GA) wide_store<!TA, TM, LA, WK>(As0 + buf * (WK * LA), tid + 256 * h, ra[h]);
+        if (GA % 256 == 0 || tid + 256 * h < GA) wide_store<!TA, TM, LA, WK>(As0 + buf * (WK * LA), tid + 256 * h, xa[h]);
 #pragma unroll
       for (int h = 0; h < HB; ++h)
-        if (GB % 256 == 0 || tid + 256 * h < GB) wide_store<TB, TN, LB, WK>(Bs0 + buf * (WK * LB), tid + 256 * h, rb[h]);
+        if (GB % 256 == 0 || tid + 256 * h < GB) wide_store<TB, TN, LB, WK>(Bs0 + buf * (WK * LB), tid + 256 * h, xb[h]);
     }
     __syncthreads();
-    if (k0 + WK < kend) {
-      if constexpr (KS) advance(k0 + WK);
-#pragma unroll
-      for (int h = 0; h < HA; ++h)
-        if (GA % 256 == 0 || tid + 256 * h < GA) ra[h] = load_a(k0 + WK, h);
-#pragma unroll
-      for (int h = 0; h < HB; ++h)
-        if (GB % 256 == 0 || tid + 256 * h < GB) rb[h] = load_b(k0 + WK, h);
-    }
+    if (more) fetch(k0 + PF * WK, xa, xb);
     if constexpr (H) {
       const _Float16* ah = Ah0 + buf * (TM * PH) + (wm + (lane & 15)) * PH + 8 * (lane >> 4);
       const _Float16* bh = Bh0 + buf * (TN * PH) + (wn + (lane & 15)) * PH + 8 * (lane >> 4);
@@ -322,26 +339,30 @@ __global__ __launch_bounds__(256) void k_gemm_w(GemmPtrs ptrs, int64_t M, int64_
 #pragma unroll
           for (int j = 0; j < WN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], b[j], acc[i][j], 0, 0, 0);
       }
-      buf = NB == 2 ? buf ^ 1 : 0;
-      continue;
+      return;
     }
     const float* as = As0 + buf * (WK * LA);
     const float* bs = Bs0 + buf * (WK * LB);
+    // Every fragment of the tile first, then the products: read by read the LDS latency came three
+    // times a tile.
+    float a[WK / 4][WM], b[WK / 4][WN];
 #pragma unroll
     for (int kk = 0; kk < WK; kk += 4) {
       // A is KC unless TA, B when TB: their columns carry the swizzle of k = kk .. kk + 3.
       const int swa = !TA ? kc_swizzle<WK>(kk) : 0, swb = TB ? kc_swizzle<WK>(kk) : 0;
       const int ka = (kk + (lane >> 4)) * LA, kb = (kk + (lane >> 4)) * LB;
-      float a[WM], b[WN];
 #pragma unroll
-      for (int i = 0; i < WM; ++i) a[i] = as[ka + ((wm + 16 * i + (lane & 15)) ^ swa)];
+      for (int i = 0; i < WM; ++i) a[kk / 4][i] = as[ka + ((wm + 16 * i + (lane & 15)) ^ swa)];
 #pragma unroll
-      for (int j = 0; j < WN; ++j) b[j] = bs[kb + ((wn + 16 * j + (lane & 15)) ^ swb)];
+      for (int j = 0; j < WN; ++j) b[kk / 4][j] = bs[kb + ((wn + 16 * j + (lane & 15)) ^ swb)];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int kk = 0; kk < WK / 4; ++kk)
 #pragma unroll
       for (int i = 0; i < WM; ++i)
 #pragma unroll
-        for (int j = 0; j < WN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
+        for (int j = 0; j < WN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[kk][i], b[kk][j], acc[i][j], 0, 0, 0);
     if (sums) {
       const float* ss = sum_a ? as : bs;
       for (int j = 0; j < sum_per; ++j) {
@@ -349,7 +370,22 @@ __global__ __launch_bounds__(256) void k_gemm_w(GemmPtrs ptrs, int64_t M, int64_
         csum += ss[kr * sum_ld + (sum_kc ? sum_col ^ kc_swizzle<WK>(kr) : sum_col)];
       }
     }
-    buf = NB == 2 ? buf ^ 1 : 0;
+  };
+  int64_t k0 = kbeg;
+  if constexpr (PF > 1) {
+    // Rounds of PF tiles whose successors all exist: their loads need no branch, across which the
+    // compiler would wait for more of them than it must.
+    for (; k0 + (2 * PF - 1) * WK < kend; k0 += PF * WK) {
+#pragma unroll
+      for (int u = 0; u < PF; ++u) tile(k0 + u * WK, u & 1, ra[u], rb[u], true);
+    }
+    for (; k0 < kend; k0 += PF * WK) {
+#pragma unroll
+      for (int u = 0; u < PF; ++u)
+        if (k0 + u * WK < kend) tile(k0 + u * WK, u & 1, ra[u], rb[u], k0 + (PF + u) * WK < kend);
+    }
+  } else {
+    for (int buf = 0; k0 < kend; k0 += WK, buf = NB == 2 ? buf ^ 1 : 0) tile(k0, buf, ra[0], rb[0], k0 + WK < kend);
   }
   if (sums) {
     __syncthreads();

@@ -233,3 +233,48 @@ def test_each_step_reads_its_own_inputs(ctx):
         got.append(np.array(losses))
     assert len(set(got[0].tolist())) == 11
     assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False)])
+@pytest.mark.parametrize("m,n", [(33, 40), (700, 36), (1030, 260)])  # tiles of 32 x 32, partial; of 32 x 64
+@pytest.mark.parametrize("k", [4, 32, 36, 96, 128, 160, 224, 256, 292, 30])  # 1 to 10 K tiles, tails, unaligned
+def test_gemm_of_few_and_many_k_tiles(ctx, m, n, k, ta, tb):
+    """K tiles fewer and more than those in flight, against float64 (2e-6 of the sum of |terms|, 292 half
+    units of 2^-24 growing as their root: f32 accumulation)."""
+    rng = np.random.default_rng(k)
+    a = rng.standard_normal((k, m) if ta else (m, k)).astype(np.float32)
+    b = rng.standard_normal((n, k) if tb else (k, n)).astype(np.float32)
+    p = Prog()
+    ai, bi = p.input("a", a.shape), p.input("b", b.shape)
+    lhs = p.op("Transpose", [ai], (m, k)) if ta else ai
+    rhs = p.op("Transpose", [bi], (k, n)) if tb else bi
+    p.out(p.op("MatMul", [lhs, rhs], (m, n)))
+    prog = ctx.program(p.text())
+    prog.run({"a": a, "b": b})
+    got = prog.output(0, m * n).reshape(m, n)
+    A, B = (a.T if ta else a).astype(np.float64), (b.T if tb else b).astype(np.float64)
+    worst = np.max(np.abs(got - A @ B) / (2e-6 * (np.abs(A) @ np.abs(B)) + 1e-30))
+    assert worst <= 1.0, worst
+
+
+@pytest.mark.parametrize("rows,v", [(1, 4), (65, 256), (17, 1023), (33, 2048), (70, 2052), (40, 4096), (2500, 64), (8, 4100),
+                                    (5, 8192), (9, 8196), (16, 2049)])
+def test_cross_entropy_of_row_blocks(ctx, oracle, rows, v):
+    """Loss and gradient at the edges of the row blocks' class counts, with more rows than blocks, odd
+    class counts, zero weights and -inf logits, against the oracle."""
+    rng = np.random.default_rng(v)
+    x = (rng.standard_normal((rows, v)) * 3).astype(np.float32)
+    x[0, 1:] = -np.inf
+    labels = rng.integers(0, v, rows).astype(np.int32)
+    labels[0] = 0
+    weights = rng.choice(np.array([0.0, 1.0, 0.5], np.float32), rows)
+    weights[0] = 1.0
+    p = Prog()
+    xi, li, wi = p.input("x", (rows, v)), p.input("labels", (rows,), "i32"), p.input("weights", (rows,))
+    g = p.scalar(1.0)
+    loss = p.op("CrossEntropy", [xi, li, wi], ())
+    p.out(loss, p.op("CrossEntropyGrad", [xi, li, wi, g], (rows, v)))
+    got, want = both(ctx, oracle, p, {"x": x, "labels": labels, "weights": weights}, (0, 1))
+    for a, b in zip(got, want):
+        ok, worst = within(a, b, np.abs(b) + 1e-6)
+        assert ok, worst
