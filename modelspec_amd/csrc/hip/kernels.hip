@@ -1104,107 +1104,32 @@ void ce_grad(hipStream_t s, const float* logits, const int32_t* labels, const fl
   MSX_LAUNCH(k_ce_grad, grid, dim3(256), 0, s, logits, labels, w, stats, den, g, o, v, ld);
 }
 
-// Cross-entropy of whole rows in one pass over the logits: a block of kCeThreads holds its row in
+// Cross-entropy of whole rows in one pass over the logits: a block of T threads holds its row in
 // registers (NV float4 a thread), takes the max and the sum of exp, writes them to stats, the
 // row's loss term max + log(sum) - x[label] to rowloss (when non-null) and, when grad is
 // non-null, the gradient g w / den (exp(x - max) / sum - onehot), the quotient taken as a product
 // with the reciprocal of the sum, zero in the padding columns. den is formed in each block exactly
 // as k_ce_loss forms it.
-constexpr int kCeThreads = 1024;
-template <int NV>
-__global__ __launch_bounds__(kCeThreads) void k_ce_rows(const float* __restrict__ x, const int32_t* __restrict__ labels,
-                                                        const float* __restrict__ w, const float* __restrict__ g,
-                                                        float* __restrict__ stats, float* __restrict__ rowloss,
-                                                        float* __restrict__ grad, int64_t rows, int64_t v, int64_t ld) {
-  constexpr int W = kCeThreads / 64;
-  __shared__ float red[W];
-  __shared__ double dred[256];
-  const int64_t r = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const float4* row = reinterpret_cast<const float4*>(x + r * ld);
-  const int64_t nq = (v + 3) / 4;
-  float e[NV][4];
-#pragma unroll
-  for (int u = 0; u < NV; ++u) {
-    const int64_t q = tid + int64_t(kCeThreads) * u;
-    const float4 f = row[q < nq ? q : nq - 1];
-    e[u][0] = f.x; e[u][1] = f.y; e[u][2] = f.z; e[u][3] = f.w;
-  }
-  auto col = [&](int u, int c) { return 4 * (tid + int64_t(kCeThreads) * u) + c; };
-  float m = -INFINITY;
-#pragma unroll
-  for (int u = 0; u < NV; ++u)
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-      if (col(u, c) < v) m = fmaxf(m, e[u][c]);
-  m = wave_max(m);
-  if (lane == 0) red[wave] = m;
-  __syncthreads();
-  m = red[0];
-#pragma unroll
-  for (int i = 1; i < W; ++i) m = fmaxf(m, red[i]);
-  __syncthreads();
-  float sum = 0.0f;
-#pragma unroll
-  for (int u = 0; u < NV; ++u)
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      e[u][c] = col(u, c) < v ? expf(e[u][c] - m) : 0.0f;
-      sum += e[u][c];
-    }
-  sum = wave_sum(sum);
-  if (lane == 0) red[wave] = sum;
-  __syncthreads();
-  float total = 0.0f;
-#pragma unroll
-  for (int i = 0; i < W; i += 2) total += red[i] + red[i + 1];
-  const int32_t lab = labels[r];
-  if (tid == 0) {
-    stats[2 * r] = m;
-    stats[2 * r + 1] = total;
-    if (rowloss) rowloss[r] = m + logf(total) - ((lab >= 0 && lab < v) ? x[r * ld + lab] : 0.0f);
-  }
-  if (!grad) return;
-  double dd = 0.0;
-  if (tid < 256)
-    for (int64_t i = tid; i < rows; i += 256) dd += double(w[i]);
-  if (tid < 256) dred[tid] = dd;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (tid < o) dred[tid] += dred[tid + o];
-    __syncthreads();
-  }
-  const float d = float(dred[0]);
-  const float scale = d == 0.0f ? 0.0f : g[0] * w[r] / d, inv = 1.0f / total;
-  float4* out = reinterpret_cast<float4*>(grad + r * ld);
-  auto gv = [&](int u, int c) {
-    const int64_t cc = col(u, c);
-    if (cc >= v || d == 0.0f) return 0.0f;
-    return scale * (e[u][c] * inv - (cc == lab ? 1.0f : 0.0f));
-  };
-#pragma unroll
-  for (int u = 0; u < NV; ++u) {
-    const int64_t q = tid + int64_t(kCeThreads) * u;
-    if (q < nq) out[q] = make_float4(gv(u, 0), gv(u, 1), gv(u, 2), gv(u, 3));
-  }
-}
-
-// The same, persistent: a block (the grid holds two for each CU) walks rows blockIdx.x,
+//
+// Persistent: a block (the grid holds two for each CU, eight of T = 256) walks rows blockIdx.x,
 // + gridDim.x, ..., the next row's loads in flight while the current row is reduced and its
 // gradient written (rows of 30522 classes: a block alone on its CU otherwise waits out each row's
-// load latency between its reductions). The weight sum is taken once a block.
-template <int NV>
-__global__ __launch_bounds__(kCeThreads) void k_ce_rows_p(const float* __restrict__ x, const int32_t* __restrict__ labels,
-                                                          const float* __restrict__ w, const float* __restrict__ g,
-                                                          float* __restrict__ stats, float* __restrict__ rowloss,
-                                                          float* __restrict__ grad, int64_t rows, int64_t v, int64_t ld) {
-  constexpr int W = kCeThreads / 64;
+// load latency between its reductions). The weight sum is taken once a block. Rows of up to 8192
+// classes take blocks of 256 threads: four barriers of 16 waves a row cost more than the row
+// (4096 rows of 4096 classes, 134 MB: 55 us with 1024 threads, 31 with 256; a wave a row 88).
+constexpr int kCeThreads = 1024;
+template <int NV, int T>
+__global__ __launch_bounds__(T) void k_ce_rows_p(const float* __restrict__ x, const int32_t* __restrict__ labels,
+                                                 const float* __restrict__ w, const float* __restrict__ g,
+                                                 float* __restrict__ stats, float* __restrict__ rowloss,
+                                                 float* __restrict__ grad, int64_t rows, int64_t v, int64_t ld) {
+  constexpr int W = T / 64;
   __shared__ float redm[W], reds[W];
   __shared__ double dred[256];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // Columns in 32 bits (v < 2^31 is checked by the launcher).
   const int nq = int((v + 3) / 4), vi = int(v);
-  auto col = [&](int u, int c) { return 4 * (tid + kCeThreads * u) + c; };
+  auto col = [&](int u, int c) { return 4 * (tid + T * u) + c; };
   float d = 0.0f;
   if (grad) {
     double dd = 0.0;
@@ -1226,7 +1151,7 @@ __global__ __launch_bounds__(kCeThreads) void k_ce_rows_p(const float* __restric
     const v4f* row = reinterpret_cast<const v4f*>(x + r * ld);
 #pragma unroll
     for (int u = 0; u < NV; ++u) {
-      const int q = tid + kCeThreads * u;
+      const int q = tid + T * u;
       const v4f f = row[q < nq ? q : nq - 1];
 #pragma unroll
       for (int c = 0; c < 4; ++c) e[u][c] = 4 * q + c < vi ? f[c] : -INFINITY;
@@ -1277,7 +1202,7 @@ __global__ __launch_bounds__(kCeThreads) void k_ce_rows_p(const float* __restric
       v4f* out = reinterpret_cast<v4f*>(grad + r * ld);
 #pragma unroll
       for (int u = 0; u < NV; ++u) {
-        const int q = tid + kCeThreads * u;
+        const int q = tid + T * u;
         v4f o;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
@@ -1365,11 +1290,14 @@ void ce_rows(hipStream_t s, const float* logits, const int32_t* labels, const fl
   // Two blocks a CU's worth of blocks: on BERT-tiny's 832 rows the graph-launched step takes 3 us
   // less than with one (0.798 against 0.801 ms, A/B alternated on one box), four 3 us more.
   const unsigned blocks = unsigned(std::min<int64_t>(rows, 2 * int64_t(cu_count())));
-#define MSX_CER(NV) MSX_LAUNCH(k_ce_rows_p<NV>, dim3(blocks), dim3(kCeThreads), 0, s, logits, labels, w, g, \
-                                       stats, rowloss, grad, rows, v, ld)
-  if (per <= 2) MSX_CER(2);
-  else if (per <= 4) MSX_CER(4);
-  else MSX_CER(8);
+#define MSX_CER(NV, T, BLOCKS)                                                                                      \
+  MSX_LAUNCH((k_ce_rows_p<NV, T>), dim3(BLOCKS), dim3(T), 0, s, logits, labels, w, g, stats, rowloss, grad, rows, v, ld)
+  const unsigned small = unsigned(std::min<int64_t>(rows, 8 * int64_t(cu_count())));
+  if (v <= 2048) MSX_CER(2, 256, small);
+  else if (v <= 4096) MSX_CER(4, 256, small);
+  else if (v <= 8192) MSX_CER(8, 256, small);
+  else if (per <= 4) MSX_CER(4, kCeThreads, blocks);
+  else MSX_CER(8, kCeThreads, blocks);
 #undef MSX_CER
 }
 
