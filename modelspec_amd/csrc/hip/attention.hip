@@ -806,7 +806,8 @@ template <int D, int T, int W>
 __global__ __launch_bounds__(64 * W) void k_attn_fwd_h16(const float* __restrict__ q, const float* __restrict__ k,
                                                          const float* __restrict__ v, const float* __restrict__ mask,
                                                          float* __restrict__ o, float* __restrict__ stats, int L, int S,
-                                                         int H, int heads, float scale) {
+                                                         int H, int heads, float scale,
+                                                         _Float16* __restrict__ o16) {
   constexpr int KP = D + 8, VP = T + 8, U = T / 16, NT = 64 * W, PT = tile_groups<D, T, NT>();
   static_assert(NT >= T, "a thread a row of the mask");
   extern __shared__ float sm[];
@@ -900,7 +901,11 @@ __global__ __launch_bounds__(64 * W) void k_attn_fwd_h16(const float* __restrict
     const float row_total = __shfl(l, 4 * g + r, 64);
     const int64_t orow = (int64_t(b) * L + i0 + 4 * g + r) * H + head * D;
 #pragma unroll
-    for (int ct = 0; ct < D / 16; ++ct) o[orow + ct * 16 + c] = oacc[ct][r] / row_total;
+    for (int ct = 0; ct < D / 16; ++ct) {
+      const float t = oacc[ct][r] / row_total;
+      o[orow + ct * 16 + c] = t;
+      if (o16) o16[orow + ct * 16 + c] = _Float16(t);
+    }
   }
   if (stats && g == 0) {
     const int64_t at = (int64_t(blockIdx.x) * L + i0 + c) * 2;
@@ -915,7 +920,8 @@ __global__ __launch_bounds__(64 * W) void k_attn_bwd_q_h16(const float* __restri
                                                            const float* __restrict__ o, const float* __restrict__ stats,
                                                            const float* __restrict__ go, float* __restrict__ dq,
                                                            float* __restrict__ dsum, int L, int S, int H, int heads,
-                                                           float scale) {
+                                                           float scale,
+                                                           _Float16* __restrict__ dq16) {
   constexpr int KP = D + 8, VP = T + 8, U = T / 16, NT = 64 * W, PT = tile_groups<D, T, NT>();
   static_assert(NT >= T, "a thread a row of the mask");
   extern __shared__ float sm[];
@@ -1005,7 +1011,11 @@ __global__ __launch_bounds__(64 * W) void k_attn_bwd_q_h16(const float* __restri
   for (int r = 0; r < 4; ++r) {
     const int64_t orow = (int64_t(b) * L + i0 + 4 * g + r) * H + head * D;
 #pragma unroll
-    for (int ct = 0; ct < D / 16; ++ct) dq[orow + ct * 16 + c] = acc[ct][r] * scale;
+    for (int ct = 0; ct < D / 16; ++ct) {
+      const float t = acc[ct][r] * scale;
+      dq[orow + ct * 16 + c] = t;
+      if (dq16) dq16[orow + ct * 16 + c] = _Float16(t);
+    }
   }
 }
 
@@ -1015,7 +1025,9 @@ __global__ __launch_bounds__(64 * W) void k_attn_bwd_kv_h16(const float* __restr
                                                             const float* __restrict__ stats, const float* __restrict__ go,
                                                             const float* __restrict__ dsum, float* __restrict__ dk,
                                                             float* __restrict__ dv, int L, int S, int H, int heads,
-                                                            float scale) {
+                                                            float scale,
+                                                            _Float16* __restrict__ dk16,
+                                                            _Float16* __restrict__ dv16) {
   constexpr int KP = D + 8, VP = T + 8, U = T / 16, NT = 64 * W, PT = tile_groups<D, T, NT>();
   static_assert(NT >= T, "a thread a row of the statistics");
   extern __shared__ float sm[];
@@ -1118,8 +1130,11 @@ __global__ __launch_bounds__(64 * W) void k_attn_bwd_kv_h16(const float* __restr
     const int64_t orow = (int64_t(b) * S + jj) * H + head * D;
 #pragma unroll
     for (int ct = 0; ct < D / 16; ++ct) {
-      if (dv) dv[orow + ct * 16 + c] = keep ? dva[ct][r] : 0.0f;
-      if (dk) dk[orow + ct * 16 + c] = keep ? dka[ct][r] * scale : 0.0f;
+      const float tv = keep ? dva[ct][r] : 0.0f, tk = keep ? dka[ct][r] * scale : 0.0f;
+      if (dv) dv[orow + ct * 16 + c] = tv;
+      if (dk) dk[orow + ct * 16 + c] = tk;
+      if (dv16) dv16[orow + ct * 16 + c] = _Float16(tv);
+      if (dk16) dk16[orow + ct * 16 + c] = _Float16(tk);
     }
   }
 }
@@ -1177,25 +1192,25 @@ void launch_bwd_q(hipStream_t s, dim3 grid, bool one, const float* q, const floa
 }
 template <int D, int T, int W>
 void launch_fwd_h(hipStream_t s, dim3 grid, const float* q, const float* k, const float* v, const float* mask,
-                  float* o, float* stats, int L, int S, int H, int heads, float scale) {
+                  float* o, float* stats, int L, int S, int H, int heads, float scale, _Float16* o16) {
   const size_t lds = size_t(h16_lds_bytes<D, T>(1, 1, 1));
-  MSX_LAUNCH((k_attn_fwd_h16<D, T, W>), grid, dim3(64 * W), lds, s, q, k, v, mask, o, stats, L, S, H, heads, scale);
+  MSX_LAUNCH((k_attn_fwd_h16<D, T, W>), grid, dim3(64 * W), lds, s, q, k, v, mask, o, stats, L, S, H, heads, scale, o16);
 }
 template <int D, int T, int W>
 void launch_bwd_q_h(hipStream_t s, dim3 grid, const float* q, const float* k, const float* v, const float* mask,
                     const float* o, const float* stats, const float* g, float* dq, float* dsum, int L, int S, int H,
-                    int heads, float scale) {
+                    int heads, float scale, _Float16* dq16) {
   const size_t lds = size_t(h16_lds_bytes<D, T>(2, 1, 1));
   MSX_LAUNCH((k_attn_bwd_q_h16<D, T, W>), grid, dim3(64 * W), lds, s, q, k, v, mask, o, stats, g, dq, dsum, L, S, H,
-             heads, scale);
+             heads, scale, dq16);
 }
 template <int D, int T, int W>
 void launch_bwd_kv_h(hipStream_t s, dim3 grid, const float* q, const float* k, const float* v, const float* mask,
                      const float* stats, const float* g, const float* dsum, float* dk, float* dv, int L, int S, int H,
-                     int heads, float scale) {
+                     int heads, float scale, _Float16* dk16, _Float16* dv16) {
   const size_t lds = size_t(h16_lds_bytes<D, T>(2, 2, 3));
   MSX_LAUNCH((k_attn_bwd_kv_h16<D, T, W>), grid, dim3(64 * W), lds, s, q, k, v, mask, stats, g, dsum, dk, dv, L, S, H,
-             heads, scale);
+             heads, scale, dk16, dv16);
 }
 template <int D, int T, int W, int KS>
 void launch_bwd_kv(hipStream_t s, dim3 grid, bool one, const float* q, const float* k, const float* v, const float* mask,
@@ -1227,6 +1242,7 @@ void launch_bwd(hipStream_t s, dim3 grid, unsigned qy, bool one, const float* q,
   }
 }  // namespace
 
+bool attention_f16(int64_t l, int64_t s) { return whole_tiles(l, s); }
 bool attention_fits(int64_t s, int64_t d) { return head_ok(d) && s <= 65535 && bwd_fits(s, s, d); }
 
 #define MSX_BY_D(d, call)                          \
@@ -1238,12 +1254,13 @@ bool attention_fits(int64_t s, int64_t d) { return head_ok(d) && s <= 65535 && b
   }
 
 void attention_fwd(hipStream_t s, const float* q, const float* k, const float* v, const float* mask, float* o,
-                   float* stats, int64_t B, int64_t L, int64_t S, int64_t H, int64_t heads, bool h16) {
+                   float* stats, int64_t B, int64_t L, int64_t S, int64_t H, int64_t heads, bool h16, _Float16* o16) {
   int64_t d = H / heads;
   if (!head_ok(d) || L > S) refuse("attention head width or query rows");
   float scale = 1.0f / sqrtf(float(d));
   if (!fwd_fits(L, S, d)) refuse("attention shape outside the kernels' LDS budget");
   h16 = h16 && whole_tiles(L, S);  // partial tiles stay in f32, also under mixed precision
+  if (o16 && !h16) refuse("an f16 attention output needs the f16 kernel");
   // 128 keys of 64-wide heads in f32 (BERT-tiny): the register-operand forward, four waves a
   // 16-query tile (8.5 us a layer against 10.0 for the LDS-staged kernel; two waves 9.9, eight
   // 9.5; the step 0.755 -> 0.751 ms). Its 16-byte loads need 16-byte aligned rows.
@@ -1255,7 +1272,7 @@ void attention_fwd(hipStream_t s, const float* q, const float* k, const float* v
   }
   const AttnPlan plan = attn_plan(B * heads, L, S, d, h16, true);
   dim3 grid(unsigned(B * heads), row_blocks(L, plan));
-#define GO_H(T, W) launch_fwd_h<D, T, W>(s, grid, q, k, v, mask, o, stats, int(L), int(S), int(H), int(heads), scale)
+#define GO_H(T, W) launch_fwd_h<D, T, W>(s, grid, q, k, v, mask, o, stats, int(L), int(S), int(H), int(heads), scale, o16)
 #define GO_F(T, W, KS) \
   launch_fwd<D, T, W, KS>(s, grid, plan.one, q, k, v, mask, o, stats, int(L), int(S), int(H), int(heads), scale)
 #define GO(D_)                                                 \
@@ -1272,12 +1289,13 @@ void attention_fwd(hipStream_t s, const float* q, const float* k, const float* v
 
 void attention_bwd(hipStream_t s, const float* q, const float* k, const float* v, const float* mask, const float* o,
                    const float* stats, const float* g, float* dq, float* dk, float* dv, float* dsum, int64_t B,
-                   int64_t L, int64_t S, int64_t H, int64_t heads, bool h16) {
+                   int64_t L, int64_t S, int64_t H, int64_t heads, bool h16, _Float16* dq16, _Float16* dk16, _Float16* dv16) {
   int64_t d = H / heads;
   if (!head_ok(d) || L > S) refuse("attention head width or query rows");
   float scale = 1.0f / sqrtf(float(d));
   if (!bwd_fits(L, S, d)) refuse("attention shape outside the kernels' LDS budget");
   h16 = h16 && whole_tiles(L, S);
+  if ((dq16 || dk16 || dv16) && !h16) refuse("f16 attention gradients need the f16 kernels");
   if (!o || !stats || !dsum) refuse("the MFMA attention backward needs the forward output and statistics");
   if (!dq) refuse("the MFMA attention backward computes d_i in its dQ pass: dQ is required");
   const AttnPlan pq = attn_plan(B * heads, L, S, d, h16, false);
@@ -1297,7 +1315,7 @@ void attention_bwd(hipStream_t s, const float* q, const float* k, const float* v
     return;
   }
 #define GO_H(T, W) \
-  launch_bwd_q_h<D, T, W>(s, gq, q, k, v, mask, o, stats, g, dq, dsum, int(L), int(S), int(H), int(heads), scale)
+  launch_bwd_q_h<D, T, W>(s, gq, q, k, v, mask, o, stats, g, dq, dsum, int(L), int(S), int(H), int(heads), scale, dq16)
 #define GO_F(T, W, KS)                                                                                            \
   launch_bwd_q<D, T, W, KS>(s, gq, pq.one, q, k, v, mask, o, stats, g, dq, dsum, int(L), int(S), int(H), int(heads), \
                           scale)
@@ -1310,7 +1328,8 @@ void attention_bwd(hipStream_t s, const float* q, const float* k, const float* v
     const AttnPlan pk = attn_plan(B * heads, S, L, d, h16, false);
     dim3 gk(unsigned(B * heads), row_blocks(S, pk));
 #define GO_H(T, W) \
-  launch_bwd_kv_h<D, T, W>(s, gk, q, k, v, mask, stats, g, dsum, dk, dv, int(L), int(S), int(H), int(heads), scale)
+  launch_bwd_kv_h<D, T, W>(s, gk, q, k, v, mask, stats, g, dsum, dk, dv, int(L), int(S), int(H), int(heads), scale, \
+                           dk16, dv16)
 #define GO_F(T, W, KS)                                                                                             \
   launch_bwd_kv<D, T, W, KS>(s, gk, pk.one, q, k, v, mask, stats, g, dsum, dk, dv, int(L), int(S), int(H), int(heads), \
                            scale)

@@ -165,6 +165,7 @@ void layer_norm(hipStream_t s, const float* x, const float* gamma, const float* 
 // `gather` ([rows] ids into the src_rows rows of a and b), row r of s is the sum's row gather[r].
 // With a_ids (b_ids), a (b) is a table of a_rows (b_rows) rows and its row r is the Embedding row
 // a_ids[r] (0 for an id out of range); not combined with `gather` or an input dropout.
+bool ln_fused_fits(int64_t rows, int64_t h);
 void ln_fused(hipStream_t s, const float* a, const float* b, const int32_t* din_token, uint64_t din_threshold,
               float din_scale, const float* gamma, const float* beta, float* s_out, float* y_out, float* stats,
               const int32_t* dout_token, uint64_t dout_threshold, float dout_scale, float* yd_out, int64_t rows,
@@ -234,12 +235,17 @@ bool attention_fits(int64_t s, int64_t d);
 // MFMA backward).
 // h16 (mixed precision): the MFMA path's contractions on the f16 MFMA with f32 accumulation.
 void attention_fwd(hipStream_t s, const float* q, const float* k, const float* v, const float* mask, float* o,
-                   float* stats, int64_t B, int64_t L, int64_t S, int64_t H, int64_t heads, bool h16 = false);
+                   float* stats, int64_t B, int64_t L, int64_t S, int64_t H, int64_t heads, bool h16 = false,
+                   _Float16* o16 = nullptr);
+// Whether h16 attention of these row counts runs in f16; its kernels then also write f16 copies of
+// their outputs where asked (o16; dq16, dk16, dv16).
+bool attention_f16(int64_t l, int64_t s);
 // Any of dk/dv may be null; the MFMA path needs dq, o (the forward's output), stats and dsum
 // ([B*heads*L] scratch).
 void attention_bwd(hipStream_t s, const float* q, const float* k, const float* v, const float* mask, const float* o,
                    const float* stats, const float* g, float* dq, float* dk, float* dv, float* dsum, int64_t B,
-                   int64_t L, int64_t S, int64_t H, int64_t heads, bool h16 = false);
+                   int64_t L, int64_t S, int64_t H, int64_t heads, bool h16 = false, _Float16* dq16 = nullptr,
+                   _Float16* dk16 = nullptr, _Float16* dv16 = nullptr);
 void prepare_attention();
 // Mixed-precision attention of 64-wide heads on the f16 operand copies (flash16.hip), for query and
 // key rows multiples of 128 (keys at most 4096): o and o16 (either may be null) the output in f32

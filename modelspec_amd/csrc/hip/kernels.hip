@@ -474,6 +474,7 @@ __global__ __launch_bounds__(256) void k_ln_fused4(const float* __restrict__ a, 
   if (stats && lane == 0) { stats[2 * row] = mean; stats[2 * row + 1] = rstd; }
 }
 
+bool ln_fused_fits(int64_t rows, int64_t h) { return h <= 1024 && rows * h <= (int64_t(1) << 32); }
 void ln_fused(hipStream_t s, const float* a, const float* b, const int32_t* din_token, uint64_t din_threshold,
               float din_scale, const float* gamma, const float* beta, float* s_out, float* y_out, float* stats,
               const int32_t* dout_token, uint64_t dout_threshold, float dout_scale, float* yd_out, int64_t rows,
@@ -483,8 +484,7 @@ void ln_fused(hipStream_t s, const float* a, const float* b, const int32_t* din_
   if (!b && !b16) bad("fused LayerNorm without its second operand");
   if (!gather) src_rows = rows;
   if ((a_ids || b_ids) && (gather || din_token)) bad("fused LayerNorm: gathered operands with a row gather or an input dropout");
-  if (h > 1024) bad("fused LayerNorm rows wider than 1024");
-  if (rows * h > (int64_t(1) << 32)) bad("fused LayerNorm over more than 2^32 elements");
+  if (!ln_fused_fits(rows, h)) bad("fused LayerNorm rows wider than 1024, or more than 2^32 elements");
   const DropoutSpec din{din_token, din_threshold, din_scale}, dout{dout_token, dout_threshold, dout_scale};
   auto al16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   if (!gather && !a_ids && !b_ids && h % 256 == 0 && h <= 1024 && al16(a) && al16(b) && al16(gamma) && al16(beta) &&

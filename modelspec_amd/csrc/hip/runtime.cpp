@@ -1515,8 +1515,17 @@ void Executor::build() {
         if (x.op == Op::LayerNorm) {
           uint32_t gm = o[1], bt = o[2];
           bool write_stats = !have;
+          // The fused kernel where its row registers hold the row (64 rows of 768: 10.3 us with the
+          // scalar kernel, 4.6 here), which also writes the f16 copy a GEMM reads (4 us of its own).
+          const bool fused = hk::ln_fused_fits(rows, h);
+          const bool y16 = fused && ld_of(id) == h && want16(id);
           push([=](hipStream_t s) {
-            hk::layer_norm(s, F(xv), F(gm), F(bt), F(id), write_stats ? static_cast<float*>(A(stats)) : nullptr, rows, h);
+            float* st2 = write_stats ? static_cast<float*>(A(stats)) : nullptr;
+            if (fused)
+              hk::ln_fused(s, nullptr, F(xv), nullptr, 0, 1.0f, F(gm), F(bt), nullptr, F(id), st2, nullptr, 0, 1.0f, nullptr,
+                           rows, h, seed, nullptr, 0, nullptr, 0, nullptr, 0, y16 ? H16(id) : nullptr);
+            else
+              hk::layer_norm(s, F(xv), F(gm), F(bt), F(id), st2, rows, h);
           });
           break;
         }
@@ -1656,11 +1665,16 @@ void Executor::build() {
           pending.back().pure = true;
           break;
         }
+        // The f16 kernels write the copies that GEMMs read themselves: a rounding launch behind each
+        // output took 3-6 us (prediction of one sequence at BERT-base's width: one a layer).
+        const bool copies16 = h16 && hk::attention_f16(L, S);
         if (x.op == Op::Attention) {
           void* st2 = R(size_t(B * heads * L) * 8);
           attn_fwd[fkey] = {id, st2};
+          const bool o16 = copies16 && ld_of(id) == H && want16(id);
           push([=](hipStream_t s) {
-            hk::attention_fwd(s, F(q), F(kv), F(v), F(mask), F(id), static_cast<float*>(A(st2)), B, L, S, H, heads, h16);
+            hk::attention_fwd(s, F(q), F(kv), F(v), F(mask), F(id), static_cast<float*>(A(st2)), B, L, S, H, heads, h16,
+                              o16 ? H16(id) : nullptr);
           });
           pending.back().pure = true;
           break;
@@ -1692,12 +1706,17 @@ void Executor::build() {
         }
         dsum = R(size_t(B * heads * L) * 4);
         if (members[0] < 0) dq_scratch = R(size_t(shape(q)[0] * H) * 4);
+        std::array<bool, 3> m16{};
+        for (int e = 0; e < 3; ++e)
+          m16[e] = copies16 && members[e] >= 0 && ld_of(uint32_t(members[e])) == H && want16(members[e]);
         push([=](hipStream_t s) {
           auto out = [&](int64_t v2) { return v2 >= 0 ? F(uint32_t(v2)) : nullptr; };
+          auto out16 = [&](int e) { return m16[e] ? H16(uint32_t(members[e])) : nullptr; };
           float* dq = members[0] >= 0 ? F(uint32_t(members[0])) : static_cast<float*>(A(dq_scratch));
           const float* fo = fwd_out >= 0 ? F(uint32_t(fwd_out)) : static_cast<float*>(A(scratch_o));
           hk::attention_bwd(s, F(q), F(kv), F(v), F(mask), fo, static_cast<float*>(A(stats_tok)), F(g), dq, out(members[1]),
-                            out(members[2]), static_cast<float*>(A(dsum)), B, L, S, H, heads, h16);
+                            out(members[2]), static_cast<float*>(A(dsum)), B, L, S, H, heads, h16, out16(0), out16(1),
+                            out16(2));
         });
         pending.back().pure = true;
         break;

@@ -278,3 +278,37 @@ def test_cross_entropy_of_row_blocks(ctx, oracle, rows, v):
     for a, b in zip(got, want):
         ok, worst = within(a, b, np.abs(b) + 1e-6)
         assert ok, worst
+
+
+@pytest.mark.parametrize("B,L,S,H,heads", [(1, 64, 64, 64, 1), (2, 48, 96, 128, 2), (3, 112, 112, 96, 3), (1, 64, 64, 768, 12),
+                                           (2, 16, 16, 200, 1), (2, 32, 32, 1040, 1), (2, 33, 33, 64, 1)])
+def test_mixed_products_of_attention_and_layer_norm(mixed, B, L, S, H, heads):
+    """A product of each of attention's output, its gradients and a LayerNorm reads the f16 rounding of
+    the f32 value beside it (1e-5 of the sum of |terms|), whether its producer writes the copy or not.
+    Head widths without a kernel: the LayerNorm alone."""
+    rng = np.random.default_rng(H)
+    fits = H // heads in (16, 32, 64, 128)
+    rows_s = {"q": B * L, "k": B * S, "v": B * S, "G": B * L}
+    inputs = {n: rng.standard_normal((r, H)).astype(np.float32) * 0.5 for n, r in rows_s.items()}
+    inputs["mask"] = np.ones((B, S), np.float32)
+    inputs["w"] = rng.standard_normal((H, 24)).astype(np.float32)
+    inputs["gamma"], inputs["beta"] = (rng.standard_normal(H).astype(np.float32) for _ in range(2))
+    p = Prog()
+    ids = {n: p.input(n, a.shape) for n, a in inputs.items()}
+    values = [(p.op("LayerNorm", [ids["q"], ids["gamma"], ids["beta"]], (B * L, H)), B * L)]
+    if fits:
+        attr = f"[heads = {heads}]"
+        operands = [ids[n] for n in ("q", "k", "v", "mask")]
+        values.append((p.op("Attention", operands, (B * L, H), attr), B * L))
+        for op, rows in (("AttentionGradQ", B * L), ("AttentionGradK", B * S), ("AttentionGradV", B * S)):
+            values.append((p.op(op, operands + [ids["G"]], (rows, H), attr), rows))
+    products = [p.op("MatMul", [v, ids["w"]], (rows, 24)) for v, rows in values]
+    p.out(*[v for v, _ in values], *products)
+    prog = mixed.program(p.text())
+    prog.run(inputs)
+    w = f16(inputs["w"])
+    for e, (_, rows) in enumerate(values):
+        value = f16(prog.output(e, rows * H).reshape(rows, H))
+        got = prog.output(len(values) + e, rows * 24).reshape(rows, 24)
+        worst = np.max(np.abs(got - value @ w) / (1e-5 * (np.abs(value) @ np.abs(w)) + 1e-30))
+        assert worst <= 1.0, (e, worst)
