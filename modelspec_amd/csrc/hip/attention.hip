@@ -39,6 +39,9 @@ __device__ __forceinline__ v4f mfma4(float a, float b, v4f c) { return __builtin
 // (own_row) and a tile's (fetch_pair) repeat the last row; the streamed ones take no part: a key
 // past the end carries mask 0, a query past the end the maximum +inf, so that its probability is
 // exp(-inf) = 0. Rows past the end are not written.
+//   0 times an infinity or a NaN is a NaN, and a masked key's row may hold them (the reference never
+// reads it), so with partial tiles such rows, and those past the end, are zeros in LDS. Whole tiles
+// stage what they find.
 __device__ __forceinline__ int own_row(int first, int c, int rows) { return first + c < rows ? first + c : rows - 1; }
 
 // Scores of U tiles of 16 LDS rows R against the 16 columns whose operand fragments xb a lane
@@ -64,7 +67,8 @@ __device__ __forceinline__ void score_tiles(const float* R, const float (&xb)[D 
 // through registers: fetch_pair issues the global loads (rows past n repeat row n - 1), put_pair
 // stores them as tiles of row stride D + 4. NT threads take part, PT = tile_groups 4-float groups
 // of each slice a thread, held as native vectors (a float4 struct array is copied through private
-// memory).
+// memory). With `partial`, put_pair stores zeros for the groups whose `lv` is 0: rows past n and, of
+// keys, those whose mask `live` is 0.
 template <int D, int T, int NT>
 constexpr int tile_groups() { return (T * (D / 4) + NT - 1) / NT; }
 template <int D, int T, int NT, int PT>
@@ -84,8 +88,27 @@ __device__ __forceinline__ void fetch_pair(v4f (&xv)[PT], v4f (&yv)[PT], const f
   }
 }
 template <int D, int T, int NT, int PT>
-__device__ __forceinline__ void put_pair(float* X, float* Y, const v4f (&xv)[PT], const v4f (&yv)[PT]) {
+__device__ __forceinline__ void fetch_pair(v4f (&xv)[PT], v4f (&yv)[PT], float (&lv)[PT], const float* __restrict__ xs,
+                                           const float* __restrict__ ys, int64_t H, int n, bool partial,
+                                           const float* __restrict__ live) {
+  fetch_pair<D, T, NT>(xv, yv, xs, ys, H, n);
+  if (partial) {
+#pragma unroll
+    for (int p = 0; p < PT; ++p) {
+      const int row = (int(threadIdx.x) + NT * p) / (D / 4);
+      lv[p] = row >= n ? 0.0f : live ? live[row] : 1.0f;
+    }
+  }
+}
+template <int D, int T, int NT, int PT>
+__device__ __forceinline__ void put_pair(float* X, float* Y, v4f (&xv)[PT], v4f (&yv)[PT], const float (&lv)[PT],
+                                         bool partial) {
   constexpr int DP = D + 4, Q = D / 4, G = T * Q;
+  if (partial) {
+#pragma unroll
+    for (int p = 0; p < PT; ++p)
+      if (lv[p] == 0.0f) xv[p] = yv[p] = v4f{0, 0, 0, 0};
+  }
 #pragma unroll
   for (int p = 0; p < PT; ++p) {
     const int e = int(threadIdx.x) + NT * p;
@@ -129,15 +152,17 @@ __global__ __launch_bounds__(64 * W) void k_attn_fwd_mfma(const float* __restric
 #pragma unroll
   for (int t = 0; t < D / 4; ++t) qb[t] = q[qrow + 4 * t + g];
   const float* mrow = mask + int64_t(b) * S;
+  const bool partial = L % 16 != 0 || S % 16 != 0;
   constexpr int NT = 64 * W, PT = tile_groups<D, T, NT>();
   static_assert(NT >= T, "a thread a row of the mask");
   const int ntiles = (S + T - 1) / T;
   const int tid = int(threadIdx.x);
   {
     v4f kv[PT], vv[PT];
-    fetch_pair<D, T, NT>(kv, vv, k + kbase, v + kbase, H, S < T ? S : T);
+    float lv[PT];
+    fetch_pair<D, T, NT>(kv, vv, lv, k + kbase, v + kbase, H, S < T ? S : T, partial, mrow);
     const float mv = tid < T && tid < S ? mrow[tid] : 0.0f;
-    put_pair<D, T, NT>(Kb, Vb, kv, vv);
+    put_pair<D, T, NT>(Kb, Vb, kv, vv, lv, partial);
     if (tid < T) Mb[tid] = mv;
   }
   __syncthreads();
@@ -150,9 +175,10 @@ __global__ __launch_bounds__(64 * W) void k_attn_fwd_mfma(const float* __restric
     const bool more = t + 1 < ntiles;
     v4f kv[PT], vv[PT];
     float mv = 0.0f;
+    float lv[PT];
     if (more) {
       const int s1 = s0 + T, n1 = S - s1 < T ? S - s1 : T;
-      fetch_pair<D, T, NT>(kv, vv, k + kbase + int64_t(s1) * H, v + kbase + int64_t(s1) * H, H, n1);
+      fetch_pair<D, T, NT>(kv, vv, lv, k + kbase + int64_t(s1) * H, v + kbase + int64_t(s1) * H, H, n1, partial, mrow + s1);
       if (tid < T && tid < n1) mv = mrow[s1 + tid];
     }
     const int nt = std::min(U, (n + 15) / 16 - half * U);
@@ -174,6 +200,8 @@ __global__ __launch_bounds__(64 * W) void k_attn_fwd_mfma(const float* __restric
       // No unmasked key yet (mn = -inf): nothing has accumulated, nothing to rescale.
       const float alpha = mn == -INFINITY ? 1.0f : expf(m - mn);
       m = mn;
+      // Live scores of -inf alone so far have exp(-inf - 0) = 0, where exp(-inf - m) is NaN.
+      const float mref = mn == -INFINITY ? 0.0f : mn;
       l *= alpha;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -187,7 +215,7 @@ __global__ __launch_bounds__(64 * W) void k_attn_fwd_mfma(const float* __restric
         float p[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          p[r] = Ms[16 * u + 4 * g + r] != 0.0f ? expf(acc[u][r] * scale - m) : 0.0f;
+          p[r] = Ms[16 * u + 4 * g + r] != 0.0f ? expf(acc[u][r] * scale - mref) : 0.0f;
           l += p[r];
         }
 #pragma unroll
@@ -199,7 +227,7 @@ __global__ __launch_bounds__(64 * W) void k_attn_fwd_mfma(const float* __restric
       }
     }
     if (more) {
-      put_pair<D, T, NT>(Kb + (j ^ 1) * 2 * T * DP, Vb + (j ^ 1) * 2 * T * DP, kv, vv);
+      put_pair<D, T, NT>(Kb + (j ^ 1) * 2 * T * DP, Vb + (j ^ 1) * 2 * T * DP, kv, vv, lv, partial);
       if (tid < T) Mb[(j ^ 1) * T + tid] = mv;
     }
     __syncthreads();
@@ -437,15 +465,17 @@ __device__ __forceinline__ void attn_bwd_q_body(const float* __restrict__ q, con
 #pragma unroll
   for (int t = 0; t < D / 4; ++t) { qb[t] = q[row + 4 * t + g]; gb[t] = go[row + 4 * t + g]; }
   const float* mrow = mask + int64_t(b) * S;
+  const bool partial = L % 16 != 0 || S % 16 != 0;
   constexpr int NT = 64 * W, PT = tile_groups<D, T, NT>();
   static_assert(NT >= T, "a thread a row of the mask");
   const int ntiles = (S + T - 1) / T;
   const int tid = int(threadIdx.x);
   {
     v4f kv[PT], vv[PT];
-    fetch_pair<D, T, NT>(kv, vv, k + kbase, v + kbase, H, S < T ? S : T);
+    float lv[PT];
+    fetch_pair<D, T, NT>(kv, vv, lv, k + kbase, v + kbase, H, S < T ? S : T, partial, mrow);
     const float mv = tid < T && tid < S ? mrow[tid] : 0.0f;
-    put_pair<D, T, NT>(Kb, Vb, kv, vv);
+    put_pair<D, T, NT>(Kb, Vb, kv, vv, lv, partial);
     if (tid < T) Mb[tid] = mv;
   }
   __syncthreads();
@@ -457,9 +487,10 @@ __device__ __forceinline__ void attn_bwd_q_body(const float* __restrict__ q, con
     const bool more = t + 1 < ntiles;
     v4f kv[PT], vv[PT];
     float mv = 0.0f;
+    float lv[PT];
     if (more) {
       const int s1 = s0 + T, n1 = S - s1 < T ? S - s1 : T;
-      fetch_pair<D, T, NT>(kv, vv, k + kbase + int64_t(s1) * H, v + kbase + int64_t(s1) * H, H, n1);
+      fetch_pair<D, T, NT>(kv, vv, lv, k + kbase + int64_t(s1) * H, v + kbase + int64_t(s1) * H, H, n1, partial, mrow + s1);
       if (tid < T && tid < n1) mv = mrow[s1 + tid];
     }
     const int nt = std::min(U, (n + 15) / 16 - half * U);
@@ -488,7 +519,7 @@ __device__ __forceinline__ void attn_bwd_q_body(const float* __restrict__ q, con
       }
     }
     if (more) {
-      put_pair<D, T, NT>(Kb + (j ^ 1) * 2 * T * DP, Vb + (j ^ 1) * 2 * T * DP, kv, vv);
+      put_pair<D, T, NT>(Kb + (j ^ 1) * 2 * T * DP, Vb + (j ^ 1) * 2 * T * DP, kv, vv, lv, partial);
       if (tid < T) Mb[(j ^ 1) * T + tid] = mv;
     }
     __syncthreads();
@@ -559,6 +590,7 @@ __device__ __forceinline__ void attn_bwd_kv_body(const float* __restrict__ q, co
 #pragma unroll
   for (int t = 0; t < D / 4; ++t) { kb[t] = k[krow + 4 * t + g]; vb[t] = v[krow + 4 * t + g]; }
   const int64_t sbase = int64_t(blockIdx.x) * L;
+  const bool partial = L % 16 != 0;
   constexpr int NT = 64 * W, PT = tile_groups<D, T, NT>();
   static_assert(NT >= T, "a thread a row of the statistics");
   const int ntiles = (L + T - 1) / T;
@@ -573,7 +605,7 @@ __device__ __forceinline__ void attn_bwd_kv_body(const float* __restrict__ q, co
     if (tid < T) {
       const int64_t at = sbase + l0 + (tid < n ? tid : n - 1);
       e[0] = tid < n ? stats[2 * at] : INFINITY;
-      e[1] = stats[2 * at + 1];
+      e[1] = tid < n ? stats[2 * at + 1] : 1.0f;
     }
 #pragma unroll
     for (int pd = 0; pd < PD; ++pd) {
@@ -593,7 +625,7 @@ __device__ __forceinline__ void attn_bwd_kv_body(const float* __restrict__ q, co
         a += __shfl_xor(a, 1, 64);
         a += __shfl_xor(a, 2, 64);
       }
-      e[2 + pd] = a;
+      e[2 + pd] = rr < n ? a : 0.0f;
     }
   };
   auto put_stats = [&](float* X, const float (&e)[2 + PD]) {
@@ -610,9 +642,10 @@ __device__ __forceinline__ void attn_bwd_kv_body(const float* __restrict__ q, co
   {
     v4f qv[PT], gv[PT];
     float e[2 + PD] = {};
-    fetch_pair<D, T, NT>(qv, gv, q + qbase, go + qbase, H, L < T ? L : T);
+    float lv[PT];
+    fetch_pair<D, T, NT>(qv, gv, lv, q + qbase, go + qbase, H, L < T ? L : T, partial, nullptr);
     fetch_stats(e, 0, L < T ? L : T);
-    put_pair<D, T, NT>(Qb, Gb, qv, gv);
+    put_pair<D, T, NT>(Qb, Gb, qv, gv, lv, partial);
     put_stats(Sb, e);
   }
   __syncthreads();
@@ -624,9 +657,10 @@ __device__ __forceinline__ void attn_bwd_kv_body(const float* __restrict__ q, co
     const bool more = t + 1 < ntiles;
     v4f qv[PT], gv[PT];
     float e[2 + PD] = {};
+    float lv[PT];
     if (more) {
       const int l1 = l0 + T, n1 = L - l1 < T ? L - l1 : T;
-      fetch_pair<D, T, NT>(qv, gv, q + qbase + int64_t(l1) * H, go + qbase + int64_t(l1) * H, H, n1);
+      fetch_pair<D, T, NT>(qv, gv, lv, q + qbase + int64_t(l1) * H, go + qbase + int64_t(l1) * H, H, n1, partial, nullptr);
       fetch_stats(e, l1, n1);
     }
     const int nt = std::min(U, (n + 15) / 16 - half * U);
@@ -660,7 +694,7 @@ __device__ __forceinline__ void attn_bwd_kv_body(const float* __restrict__ q, co
       }
     }
     if (more) {
-      put_pair<D, T, NT>(Qb + (j ^ 1) * 2 * T * DP, Gb + (j ^ 1) * 2 * T * DP, qv, gv);
+      put_pair<D, T, NT>(Qb + (j ^ 1) * 2 * T * DP, Gb + (j ^ 1) * 2 * T * DP, qv, gv, lv, partial);
       put_stats(Sb + (j ^ 1) * 3 * T, e);
     }
     __syncthreads();

@@ -57,6 +57,41 @@ def test_attention_over_partial_tiles(ctx, oracle, B, L, S, H, heads, mixed):
         assert np.all(g.reshape(B * S, H)[mask.reshape(-1) == 0] == 0)
 
 
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("B,L,S,H,heads", [(2, 17, 17, 64, 1), (3, 100, 100, 192, 3), (1, 150, 150, 64, 1), (2, 20, 48, 64, 2),
+                                           (2, 33, 33, 128, 1), (2, 90, 300, 32, 2), (43, 100, 100, 224, 14)])
+def test_attention_over_partial_tiles_leaves_masked_keys_out(ctx, oracle, B, L, S, H, heads, mixed):
+    """What a masked key and its value hold (NaN, infinities) reaches no result, and a run of live keys
+    whose scores all overflow to -inf (those of a whole tile, before the first finite score) has
+    probability 0: the oracle's values, which reads unmasked keys only."""
+    rng = np.random.default_rng(S + H)
+    q, G = (rng.uniform(0.1, 1.0, (B * L, H)).astype(np.float32) for _ in range(2))
+    k, v = (rng.uniform(-1.0, 1.0, (B, S, H)).astype(np.float32) for _ in range(2))
+    mask = (rng.random((B, S)) < 0.6).astype(np.float32)
+    mask[:, S - 1] = 1.0
+    k[:, :S * 2 // 3] = -3e38
+    k[mask == 0], v[mask == 0] = np.nan, np.inf
+    v[(mask == 0) & (np.arange(S) % 2 == 0)] = np.nan
+    p = Prog()
+    qi, ki, vi = p.input("q", (B * L, H)), p.input("k", (B * S, H)), p.input("v", (B * S, H))
+    mi, Gi = p.input("mask", (B, S)), p.input("G", (B * L, H))
+    attr = f"[heads = {heads}]"
+    outs = [p.op("Attention", [qi, ki, vi, mi], (B * L, H), attr)]
+    for op, rows in (("AttentionGradQ", B * L), ("AttentionGradK", B * S), ("AttentionGradV", B * S)):
+        outs.append(p.op(op, [qi, ki, vi, mi, Gi], (rows, H), attr))
+    inputs = {"q": q, "k": k.reshape(B * S, H), "v": v.reshape(B * S, H), "mask": mask, "G": G}
+    ctx.set_precision(mixed)
+    try:
+        got, want = both(ctx, oracle, p.out(*outs), inputs, (0, 1, 2, 3))
+    finally:
+        ctx.set_precision(False)
+    # |values| of at most 1: the bound of attention_case with unit magnitudes.
+    for idx, (g, w) in enumerate(zip(got, want)):
+        assert np.all(np.isfinite(w)), idx
+        ok, worst = within(g, w, np.abs(w) + 1 + 4 * np.sqrt(H // heads))
+        assert ok, (idx, worst)
+
+
 def f16(x):
     return np.asarray(x, np.float32).astype(np.float16).astype(np.float64)
 
