@@ -539,7 +539,13 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGM * WGN == 8 ? 2 : 4) void k_gemm
 }
 
 // ---------------------------------------------------------------------------------------------
-bool gemm16_layout(const GemmArgs& o) { return o.lda % 8 == 0 && o.ldb % 8 == 0; }
+// A lane's offset from its tile's first row and K is 32 bits of bytes: up to 255 rows of a KC operand,
+// 63 of another. K, in 32 bits too, is counted up to the end of its last tile.
+bool gemm16_takes(int64_t lda, bool akc, int64_t ldb, bool bkc, int64_t k) {
+  auto pitch = [](int64_t ld, bool kc) { return ld % 8 == 0 && ld <= (int64_t(1) << (kc ? 23 : 25)); };
+  return pitch(lda, akc) && pitch(ldb, bkc) && k <= INT32_MAX - 63;
+}
+bool gemm16_layout(const GemmArgs& o) { return gemm16_takes(o.lda, !o.ta, o.ldb, o.tb, o.k); }
 
 // Split-K of a mixed-precision product. A deferred one (a weight gradient, its slices summed by the
 // batched finalize) takes up to 1024 128 x 128 tiles; its slices keep 3200 K of a K of 8192 or more

@@ -102,7 +102,7 @@ bool gemm_lds(hipStream_t s, const GemmArgs& g, const GemmPtrs& ptrs, int split,
 // f16 output copies asked for.
 bool gemm16(hipStream_t s, const GemmArgs* list, int count, const GemmPtrs& ptrs, int split, int64_t chunk);
 // Whether gemm16 takes a problem of this layout (its f16 operand copies present and 16-byte aligned
-// aside): rows of whole 16-byte groups.
+// aside): gemm16_takes.
 bool gemm16_layout(const GemmArgs& g);
 // The split-K slices of a mixed-precision product.
 struct Split16 {

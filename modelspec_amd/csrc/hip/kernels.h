@@ -140,8 +140,11 @@ int64_t gemm_workspace(int64_t m, int64_t n, int64_t k, bool colsum = false, boo
 // The column_finalize jobs that finish a deferred split-K gemm (0, 1 or 2 written to jobs).
 int gemm_deferred_jobs(const GemmArgs& g, ColumnJob* jobs);
 // Whether a mixed-precision problem runs on gemm16 (gemm16.hip) once its f16 operand copies are given
-// (16-byte aligned): no cross-entropy operand, rows of whole 16-byte groups.
+// (16-byte aligned): no cross-entropy operand, and gemm16_takes its layout.
 bool gemm16_fits(const GemmArgs& g);
+// Operand rows of whole 16-byte f16 groups, pitches and K within the kernels' 32-bit offsets; akc, bkc:
+// the operand is contiguous along K.
+bool gemm16_takes(int64_t lda, bool akc, int64_t ldb, bool bkc, int64_t k);
 void gemm(hipStream_t s, const GemmArgs& g);
 // `count` (1 .. kGemmGroupMax) independent GEMMs that differ only in their pointers, in one
 // launch; split-K slices of a group are summed by deferral only.

@@ -256,7 +256,8 @@ void Executor::build() {
   // A SumRows of a MatMul's un-transposed B operand (the bias gradient beside its weight gradient)
   // is taken by that GEMM from its LDS tiles, when no reader of the sum comes before the GEMM.
   // Under mixed precision only the f16 GEMM on the operands' f16 copies (gemm16) takes the
-  // sums (of the f16 values): both operands' rows whole 16-byte groups of f16, K a multiple of 32.
+  // sums (of the f16 values). It is given them where K is a multiple of 32, though its kernels sum any
+  // K: batches of other row counts keep the separate pass, the f32 sum of the unrounded values.
   std::map<uint32_t, uint32_t> colsum_of;  // MatMul -> SumRows
   std::set<uint32_t> colsum_fused;
   const bool mixed_twins = s_.opt_.mixed && !s_.opt_.fuse_ce_head;
@@ -266,7 +267,7 @@ void Executor::build() {
     const Resolved ra = resolve(p, m.operands[0]), rb = resolve(p, m.operands[1]);
     const auto &sa = p.node(ra.src).ty.shape, &sb = p.node(rb.src).ty.shape;
     const int64_t k = p.node(m.operands[0]).ty.shape[1];
-    return sa.size() == 2 && sb.size() == 2 && sa[1] % 8 == 0 && sb[1] % 8 == 0 && k % 32 == 0;
+    return sa.size() == 2 && sb.size() == 2 && hk::gemm16_takes(sa[1], !ra.flip, sb[1], false, k) && k % 32 == 0;
   };
   for (size_t k = 0; k < n; ++k) {
     if (!need[k] || p.nodes[k].op != Op::SumRows) continue;

@@ -19,6 +19,7 @@ import pytest
 from modelspec_amd import api
 
 import kernel_ir
+from ops_lib import Prog
 
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden")
 
@@ -125,3 +126,32 @@ def test_bert_tiny_step_plan_takes_the_fused_paths():
     assert sum(w.startswith("CrossEntropyRows") for w in whats) == 1, whats
     # The EmbeddingGrad plans of the host-staged ids are made by the host with the step's inputs.
     assert not any(w.startswith("EmbeddingPlan") for w in whats), whats
+
+
+def forward_plan(p, mixed):
+    """The launch plan of a program of its own, beside any step."""
+    step_ir, _ = api.compile_config("linear_regression")
+    return kernel_ir.parse_plan(api.plan(step_ir, p.text(), 0, mixed))["forward"]
+
+
+@pytest.mark.parametrize("m,k,n,ta,tb,chained", [
+    (64, 64, 2 ** 25, False, False, True), (64, 64, 2 ** 25 + 64, False, False, False),
+    (2 ** 25, 64, 64, True, False, True), (2 ** 25 + 64, 64, 64, True, False, False),
+    (4096, 2 ** 23, 4096, False, True, True), (4096, 2 ** 23 + 64, 4096, False, True, False),
+])
+def test_mixed_products_past_32_bit_offsets_stay_off_the_f16_kernels(m, k, n, ta, tb, chained):
+    """The f16 GEMM addresses an operand's tile by 32-bit byte offsets: 63 rows of a pitch up to 2^25
+    halves where the rows run along K's columns, 255 of one up to 2^23 where they are contiguous along
+    K, so 63 (2^25 + 256) 2 and 255 2^23 2 + 128 bytes both stay below 2^32. Two products added into
+    one value join over their K only where that kernel takes them, which shows where the plan draws
+    the line; a wider pitch goes to the kernel with 64-bit addresses."""
+    p = Prog()
+    total = p.input("x", (m, n))
+    for q in (1, 2):
+        a = p.input(f"a{q}", (k, m) if ta else (m, k))
+        w = p.input(f"w{q}", (n, k) if tb else (k, n))
+        lhs = p.op("Transpose", [a], (m, k)) if ta else a
+        rhs = p.op("Transpose", [w], (k, n)) if tb else w
+        total = p.op("Add", [total, p.op("MatMul", [lhs, rhs], (m, n))], (m, n))
+    products = [l["what"] for l in forward_plan(p.out(total), True)["launches"] if l["what"].startswith("MatMul")]
+    assert len(products) == (1 if chained else 2) and (" (+) " in products[0]) == chained, products
