@@ -32,7 +32,7 @@ __device__ __forceinline__ v4f mfma4(float a, float b, v4f c) { return __builtin
 // MFMAs, and one barrier a tile hands the buffers over. Row stride of every LDS tile is D + 4
 // floats: the 16 rows x 4 columns an MFMA operand read touches fall in distinct banks.
 
-// The f32 kernels take any row count; one that is no multiple of 16 leaves a partial last tile. A
+// In the f32 kernels a row count that is no multiple of 16 leaves a partial last tile. A
 // scalar kernel (one thread a row, a head a block) took such sequences before: 2186 us backward and
 // 158 us forward a layer for 36 heads of 100 x 64, every row walking all keys serially, against
 // 18.1 and 10.2 us here. A wave's own rows past the end
@@ -1175,8 +1175,9 @@ __global__ __launch_bounds__(64 * W) void k_attn_bwd_kv_h16(const float* __restr
 
 // ---------------------------------------------------------------------------------------------
 namespace {
-// Row counts that are no multiple of 16 are taken while a head's operands stay within one block's
-// LDS as plain f32 rows (S of at most 157 for 64-wide heads): the declared limit of such sequences.
+// Row counts that are no multiple of 16 are taken while a head's operands would fit one block's LDS as
+// plain f32 rows (self-attention of at most 157 rows for 64-wide heads): the limit of what is accepted,
+// kept from a kernel that staged them so. The kernels here stream tiles and have none.
 bool whole_tiles(int64_t L, int64_t S) { return L % 16 == 0 && S % 16 == 0; }
 bool fwd_fits(int64_t L, int64_t S, int64_t d) { return whole_tiles(L, S) || size_t(2 * S * d + S) * 4 <= kLdsMax; }
 bool bwd_fits(int64_t L, int64_t S, int64_t d) {
@@ -1277,7 +1278,9 @@ void launch_bwd(hipStream_t s, dim3 grid, unsigned qy, bool one, const float* q,
 }  // namespace
 
 bool attention_f16(int64_t l, int64_t s) { return whole_tiles(l, s); }
-bool attention_fits(int64_t s, int64_t d) { return head_ok(d) && s <= 65535 && bwd_fits(s, s, d); }
+bool attention_fits(int64_t l, int64_t s, int64_t d, bool gradient) {
+  return head_ok(d) && s <= 65535 && bwd_fits(s, s, d) && (gradient ? bwd_fits(l, s, d) : fwd_fits(l, s, d));
+}
 
 #define MSX_BY_D(d, call)                          \
   switch (d) {                                     \

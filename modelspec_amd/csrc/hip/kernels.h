@@ -232,7 +232,8 @@ void dropout(hipStream_t s, const float* x, float* o, int64_t n, const int32_t* 
              uint64_t threshold, float scale);
 
 // Attention over a key mask [B, S]; q [B*L, H], k/v [B*S, H] (attention.hip).
-bool attention_fits(int64_t s, int64_t d);
+// Whether a launch takes these row counts and head width (l query rows, s key rows a sequence).
+bool attention_fits(int64_t l, int64_t s, int64_t d, bool gradient);
 
 // stats: [B*heads*L, 2] softmax maximum and sum per query (written when non-null; required by the
 // MFMA backward).

@@ -1603,7 +1603,8 @@ void Executor::build() {
         if (p.node(o[3]).ty.dtype != DType::F32) throw IrError("attention over key spans has no HIP kernel yet");
         uint32_t q = o[0], kv = o[1], v = o[2], mask = o[3];
         int64_t B = shape(mask)[0], S = shape(mask)[1], L = shape(q)[0] / B, H = shape(q)[1], heads = x.heads;
-        if (!hk::attention_fits(S, H / heads)) throw IrError("attention shape has no HIP kernel (head width or sequence too large)");
+        if (!hk::attention_fits(L, S, H / heads, x.op != Op::Attention))
+          throw IrError("attention shape has no HIP kernel (head width, row counts or sequence too large)");
         if (p.node(mask).op == Op::Input) key_masks_.push_back(p.node(mask).name);
         auto fkey = std::vector<uint32_t>{q, kv, v, mask, uint32_t(heads)};
         const bool h16 = s_.opt_.mixed;  // mixed precision: the f16 MFMA

@@ -155,3 +155,25 @@ def test_mixed_products_past_32_bit_offsets_stay_off_the_f16_kernels(m, k, n, ta
         total = p.op("Add", [total, p.op("MatMul", [lhs, rhs], (m, n))], (m, n))
     products = [l["what"] for l in forward_plan(p.out(total), True)["launches"] if l["what"].startswith("MatMul")]
     assert len(products) == (1 if chained else 2) and (" (+) " in products[0]) == chained, products
+
+
+@pytest.mark.parametrize("L,S,H,heads,taken", [
+    (96, 512, 64, 1, "all"), (512, 512, 64, 1, "all"), (157, 157, 64, 1, "all"), (158, 158, 64, 1, "none"),
+    (100, 112, 64, 1, "all"), (100, 240, 64, 1, "forward"),  # 2 S d + S floats fit one LDS, with 2 L d + 3 L not
+    (100, 512, 64, 1, "none"), (1, 336, 64, 1, "none"), (300, 304, 16, 1, "all"), (80, 80, 24, 1, "none"),
+])
+def test_attention_row_counts_are_refused_by_the_plan(L, S, H, heads, taken):
+    """What no launch takes is refused when the program is planned, as unsupported, and not by the
+    launch (inside a step's capture): row counts that are no multiple of 16 past the size limit, also
+    where only the query rows are none."""
+    for op in ("Attention", "AttentionGradQ", "AttentionGradK", "AttentionGradV"):
+        p = Prog()
+        q, k, v = p.input("q", (L, H)), p.input("k", (S, H)), p.input("v", (S, H))
+        operands = [q, k, v, p.input("mask", (1, S))] + ([p.input("G", (L, H))] if op != "Attention" else [])
+        p.out(p.op(op, operands, (L if op in ("Attention", "AttentionGradQ") else S, H), f"[heads = {heads}]"))
+        if taken == "all" or (taken == "forward" and op == "Attention"):
+            assert any(l["what"].startswith("Attention") for l in forward_plan(p, False)["launches"]), op
+        else:
+            with pytest.raises(api.MsxError, match="no HIP kernel") as e:
+                forward_plan(p, False)
+            assert e.value.code == -5, (op, e.value.code)
