@@ -473,9 +473,13 @@ namespace {
 // The tile shape and split-K of a GEMM, from measured MI355X timings of the step's shapes: large
 // outputs (and very deep K) take 64 x 64 tiles, outputs up to 2^19 elements 32 x 32, the rest
 // 32 x 64. Split-K, whose slice sum costs a launch unless deferred to a batched finalize, is used
-// when deferred or when K is deep, to fill the chip.
+// when deferred or when K is deep, to fill the chip. A mixed-precision product is split by the kernel
+// it is planned for: gemm16 by its own rule, k_gemm_w's 128 x 128 f16 tiles (operands whose pitch is no
+// multiple of 8, or without f16 copies) to about 1024 blocks. Left unsplit as gemm16's are, which has
+// smaller tiles instead, a block of 4096 x 256 over 5003 classes took 925 us a step against 715, a
+// 512-wide encoder of FFN width 2052 988 against 810.
 struct SplitPlan { int wm, wn, wk, split; int64_t chunk; };
-SplitPlan split_plan(int64_t m, int64_t n, int64_t k, bool defer, bool h16, bool ce = false) {
+SplitPlan split_plan(int64_t m, int64_t n, int64_t k, bool defer, bool h16, bool ce, bool on16) {
   const int64_t mn = m * n;
   SplitPlan p{};
   // Mixed precision: k_gemm_w's largest f16 tile (where gemm16 does not take the problem).
@@ -484,7 +488,7 @@ SplitPlan split_plan(int64_t m, int64_t n, int64_t k, bool defer, bool h16, bool
   else if (ce || mn >= (int64_t(1) << 21) || k >= 8192) { p.wm = 2; p.wn = 2; p.wk = 16; }
   else if (mn <= (int64_t(1) << 19)) { p.wm = 1; p.wn = 1; p.wk = 32; }
   else { p.wm = 1; p.wn = 2; p.wk = 16; }
-  if (h16 && !ce) {
+  if (on16) {
     const Split16 q = gemm16_split(m, n, k, defer);
     p.split = q.split;
     p.chunk = q.chunk;
@@ -498,33 +502,35 @@ SplitPlan split_plan(int64_t m, int64_t n, int64_t k, bool defer, bool h16, bool
     // An f32 product of K 8192 or more summed by its own launch (BERT-tiny's decoder input
     // gradient, K 30522): half as many slices, 74 -> 37 (A/B in one run: 74 -> 68 us, half the
     // partials written and read back; a quarter as many 74 us, 1.5 times as many 81 us).
-    if (!defer && k >= 8192) want = std::max<int64_t>(1, want / 2);
+    if (!h16 && !defer && k >= 8192) want = std::max<int64_t>(1, want / 2);
   }
   // Deferred slices keep 128 K steps or more: their partials all go through the finalize, m n
-  // floats a slice.
-  const int64_t split = std::max<int64_t>(1, std::min(want, k / (defer ? 128 : 64)));
+  // floats a slice (512, of a K of 8192 or more 4096, for the 128 x 128 f16 tiles).
+  const int64_t deferred = p.wm == 4 ? (k >= 8192 ? 4096 : 512) : 128;
+  const int64_t split = std::max<int64_t>(1, std::min(want, k / (defer ? deferred : 64)));
   p.chunk = ((k + split - 1) / split + kSliceAlign - 1) / kSliceAlign * kSliceAlign;
   p.split = int((k + p.chunk - 1) / p.chunk);
   return p;
 }
 }  // namespace
 
-int gemm_split_for(int64_t m, int64_t n, int64_t k, bool defer, bool h16, bool ce) {
-  return split_plan(m, n, k, defer, h16, ce).split;
+int gemm_split_for(int64_t m, int64_t n, int64_t k, bool defer, bool h16, bool ce, bool on16) {
+  return split_plan(m, n, k, defer, h16, ce, on16).split;
 }
 
 int64_t gemm_tile_n(int64_t m, int64_t n, int64_t k, bool defer, bool h16) {
-  return 32 * split_plan(m, n, k, defer, h16, true).wn;
+  return 32 * split_plan(m, n, k, defer, h16, true, false).wn;
 }
 
-int64_t gemm_workspace(int64_t m, int64_t n, int64_t k, bool colsum, bool sum_a, bool defer, bool h16, bool ce) {
-  const int split = gemm_split_for(m, n, k, defer, h16, ce);
+int64_t gemm_workspace(int64_t m, int64_t n, int64_t k, bool colsum, bool sum_a, bool defer, bool h16, bool ce,
+                       bool on16) {
+  const int split = gemm_split_for(m, n, k, defer, h16, ce, on16);
   if (split <= 1) return 0;
   return int64_t(split) * m * n + (colsum ? int64_t(split) * (sum_a ? m : n) : 0);  // partials, then sums
 }
 
 int gemm_deferred_jobs(const GemmArgs& g, ColumnJob* jobs) {
-  const int split = gemm_split_for(g.m, g.n, g.k, g.defer, g.h16, g.ce_operand != 0 || g.ce_part);
+  const int split = gemm_split_for(g.m, g.n, g.k, g.defer, g.h16, g.ce_operand != 0 || g.ce_part, g.on16);
   if (split <= 1) return 0;
   if (g.bias || g.addend || g.act || g.drop_token || g.ldc != g.n) bad("deferred split-K needs a dense output without epilogue");
   if (g.m * g.n > INT32_MAX) bad("deferred split-K output too large");
@@ -552,15 +558,16 @@ void gemm_group(hipStream_t s, const GemmArgs* list, int count) {
     const GemmArgs& o = list[q];
     if (o.m != g.m || o.n != g.n || o.k != g.k || o.lda != g.lda || o.ldb != g.ldb || o.ldc != g.ldc || o.ta != g.ta ||
         o.tb != g.tb || o.sum_a != g.sum_a || o.defer != g.defer || o.pad_a != g.pad_a || o.pad_b != g.pad_b ||
-        o.pad_c != g.pad_c || o.h16 != g.h16 || o.act != g.act || (o.colsum == nullptr) != (g.colsum == nullptr) ||
+        o.pad_c != g.pad_c || o.h16 != g.h16 || o.on16 != g.on16 || o.act != g.act || (o.colsum == nullptr) != (g.colsum == nullptr) ||
         (o.bias == nullptr) != (g.bias == nullptr) || (o.addend == nullptr) != (g.addend == nullptr) ||
         (o.workspace == nullptr) != (g.workspace == nullptr) || (o.drop_token == nullptr) != (g.drop_token == nullptr))
       bad("gemm group of unlike problems");
   }
   const int ce = g.ce_part ? 3 : g.ce_operand;
-  if (ce && (count != 1 || (ce == 3 && g.k > 0 && split_plan(g.m, g.n, g.k, g.defer, g.h16, true).split > 1)))
+  if (ce && (count != 1 || (ce == 3 && g.k > 0 && split_plan(g.m, g.n, g.k, g.defer, g.h16, true, false).split > 1)))
     bad("a cross-entropy head GEMM runs alone, and its forward without split-K");
-  const SplitPlan plan = split_plan(g.m, g.n, g.k, g.defer, g.h16, ce != 0);
+  if (g.on16 && (!g.h16 || ce)) bad("gemm16 takes mixed-precision problems without a cross-entropy operand");
+  const SplitPlan plan = split_plan(g.m, g.n, g.k, g.defer, g.h16, ce != 0, g.on16);
   const int split = plan.split;
   const int ksegs = g.ksegs > 1 ? g.ksegs : 1;
   if (ksegs > 1 && (count != 1 || ksegs > kGemmGroupMax || g.k % ksegs != 0 || (g.k / ksegs) % 32 != 0 || split != 1 ||
@@ -577,7 +584,7 @@ void gemm_group(hipStream_t s, const GemmArgs* list, int count) {
     float* ws = nullptr;
     if (split > 1) {
       if (!o.workspace ||
-          o.workspace_floats < gemm_workspace(o.m, o.n, o.k, o.colsum != nullptr, o.sum_a, o.defer, o.h16, ce != 0))
+          o.workspace_floats < gemm_workspace(o.m, o.n, o.k, o.colsum != nullptr, o.sum_a, o.defer, o.h16, ce != 0, o.on16))
         bad("gemm split-K workspace too small");
       ws = o.workspace;
     }
@@ -693,11 +700,11 @@ void gemm_group(hipStream_t s, const GemmArgs* list, int count) {
   if (plan.wm == 2) MSX_KS_V(TA, TB, 2, 2, 16);             \
   else if (plan.wn == 2) MSX_KS_V(TA, TB, 1, 2, 16);        \
   else MSX_KS_V(TA, TB, 1, 1, 32);
-  // The large f32 shapes take k_gemm_lds when their layout allows it, mixed-precision GEMMs whose
-  // operands both have f16 copies the kernels of gemm16.hip.
+  // The large f32 shapes take k_gemm_lds when their layout allows it, mixed-precision GEMMs planned for
+  // them the kernels of gemm16.hip.
   bool f16_out = false;  // the launched kernel writes the f16 output copies itself
   const bool lds = !g.h16 && ksegs == 1 && count == 1 && !ce && gemm_lds(s, g, ptrs, split, chunk);
-  const bool lds16 = !lds && g.h16 && !ce && gemm16(s, list, count, ptrs, split, chunk);
+  const bool lds16 = g.on16 && gemm16(s, list, count, ptrs, split, chunk);
   if (lds16) f16_out = true;
   for (int q = 0; q < count && !lds16; ++q)
     if ((ksegs == 1 && (!list[q].a || !list[q].b)) || !list[q].c)

@@ -99,6 +99,9 @@ struct GemmArgs {
   const float* seg_b[4];
   const _Float16* seg_a16[4];  // mixed precision: the segments' f16 copies
   const _Float16* seg_b16[4];
+  // Planned for gemm16 (gemm16_fits, and the plan keeps both operands' f16 copies): its split-K, then
+  // its kernels.
+  bool on16;
 };
 enum GemmAct : int { EPI_NONE, EPI_GELU, EPI_RELU, EPI_GELU_GRAD, EPI_RELU_GRAD };
 struct GemmEpi {
@@ -131,12 +134,14 @@ struct GemmPtrs {
 // The output tile width of a GEMM of this shape (the column tiles of ce_part).
 int64_t gemm_tile_n(int64_t m, int64_t n, int64_t k, bool defer = false, bool h16 = false);
 // The split-K factor the launcher uses (with `defer` as in GemmArgs).
-// ce: a cross-entropy head GEMM (GemmArgs ce_part or ce_operand), which takes the largest tile.
-int gemm_split_for(int64_t m, int64_t n, int64_t k, bool defer = false, bool h16 = false, bool ce = false);
+// ce: a cross-entropy head GEMM (GemmArgs ce_part or ce_operand), which takes the largest tile;
+// on16 as in GemmArgs.
+int gemm_split_for(int64_t m, int64_t n, int64_t k, bool defer = false, bool h16 = false, bool ce = false,
+                   bool on16 = false);
 // Floats of workspace a gemm of this shape needs (0 without split-K): the slices' partial
 // products, then the slices' column (row) sums when asked for.
 int64_t gemm_workspace(int64_t m, int64_t n, int64_t k, bool colsum = false, bool sum_a = false, bool defer = false,
-                       bool h16 = false, bool ce = false);
+                       bool h16 = false, bool ce = false, bool on16 = false);
 // The column_finalize jobs that finish a deferred split-K gemm (0, 1 or 2 written to jobs).
 int gemm_deferred_jobs(const GemmArgs& g, ColumnJob* jobs);
 // Whether a mixed-precision problem runs on gemm16 (gemm16.hip) once its f16 operand copies are given

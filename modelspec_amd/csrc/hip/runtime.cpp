@@ -907,6 +907,10 @@ void Executor::build() {
     token16_[vid] = arena_.reserve(size_t(x.ty.shape[0] * ld_of(vid)) * 2);
     return true;
   };
+  // Whether v has one: a value's is reserved with its producer, so before the GEMMs that read it.
+  auto has16 = [&](uint32_t v) {
+    return token16_.count(v) || fixed16_.count(v) || (s_.opt_.plan_only && p.node(v).op == Op::ParamRead);
+  };
   auto H16 = [this](int64_t v) -> _Float16* { return v >= 0 ? ptr16(uint32_t(v)) : nullptr; };
   // The launch of one GEMM or a group of like GEMMs (one hk::gemm_group call).
   auto gemm_launch = [this, F, A, I](std::vector<std::shared_ptr<GemmJob>> jobs) {
@@ -1281,7 +1285,8 @@ void Executor::build() {
         int64_t bias_id = fused ? int64_t(o[1]) : -1;
         // Split-K partials only the optimizer reads are summed by the batched column finalize.
         g.defer = bias_id < 0 && epi.node == id && only_optimizer_reads(int64_t(out_id)) && only_optimizer_reads(cs_id);
-        int64_t wsf = hk::gemm_workspace(g.m, g.n, g.k, cs_id >= 0, g.sum_a, g.defer, g.h16, g.ce_operand || ce_part);
+        g.on16 = mixed_twins && !ce_part && has16(asrc) && has16(bsrc) && hk::gemm16_fits(g);
+        int64_t wsf = hk::gemm_workspace(g.m, g.n, g.k, cs_id >= 0, g.sum_a, g.defer, g.h16, g.ce_operand || ce_part, g.on16);
         void* ws = wsf > 0 ? R(size_t(wsf) * 4) : nullptr;
         g.workspace_floats = wsf;
         auto job = std::make_shared<GemmJob>();
@@ -1307,7 +1312,7 @@ void Executor::build() {
         pending.push_back({gemm_launch({job}), 0, 0, is_step_ && g.defer, {job}});
         pending.back().pure = true;
         if (g.defer && wsf > 0) {
-          const int split = hk::gemm_split_for(g.m, g.n, g.k, true, g.h16, g.ce_operand != 0);
+          const int split = hk::gemm_split_for(g.m, g.n, g.k, true, g.h16, g.ce_operand != 0, g.on16);
           const int32_t mn = int32_t(g.m * g.n);
           deferred.push_back({ws, 0, int64_t(out_id), -1, split, mn, mn});
           if (cs_id >= 0) {
@@ -1903,19 +1908,15 @@ void Executor::build() {
   // Under mixed precision the segments are read as f16 copies by gemm16, K tiles of 64 (BERT-base's
   // three 16384 x 768 x 768 products, each adding 50 MB of f32 into the next: 3 x 42 us, in one 65).
   {
-    auto has16 = [&](uint32_t v) {
-      return token16_.count(v) || fixed16_.count(v) || (s_.opt_.plan_only && p.node(v).op == Op::ParamRead);
-    };
     auto chainable = [&](const GemmJob& j) {
       return j.epi.node != j.id && j.epi.act == hk::EPI_NONE && j.bias_id < 0 && j.cs_id < 0 && !j.ws &&
              !j.ce_part && !j.ce_tab && j.segs.empty() && !j.g.defer &&
-             (j.g.h16 ? mixed_twins && j.g.k % 64 == 0 && has16(j.asrc) && has16(j.bsrc) && hk::gemm16_fits(j.g)
-                      : j.g.k % 32 == 0);
+             (j.g.h16 ? j.g.on16 && j.g.k % 64 == 0 : j.g.k % 32 == 0);
     };
     auto same = [](const hk::GemmArgs& a, const hk::GemmArgs& b) {
       return a.m == b.m && a.n == b.n && a.k == b.k && a.lda == b.lda && a.ldb == b.ldb && a.ldc == b.ldc &&
              a.ta == b.ta && a.tb == b.tb && a.pad_a == b.pad_a && a.pad_b == b.pad_b && a.pad_c == b.pad_c &&
-             a.h16 == b.h16;
+             a.h16 == b.h16 && a.on16 == b.on16;
     };
     std::vector<bool> gone(pending.size(), false);
     for (size_t i = 0; i < pending.size(); ++i) {
@@ -1926,7 +1927,7 @@ void Executor::build() {
       while (chain.size() < size_t(hk::kGemmGroupMax)) {
         const GemmJob& cur = *pending[chain.back()].gemm[0];
         if (cur.epi.drop >= 0 || consumers[p.pos.at(cur.out_id)].size() != 1) break;
-        if (hk::gemm_split_for(head.g.m, head.g.n, head.g.k * int64_t(chain.size() + 1), false, head.g.h16) != 1) break;
+        if (hk::gemm_split_for(head.g.m, head.g.n, head.g.k * int64_t(chain.size() + 1), false, head.g.h16, false, head.g.on16) != 1) break;
         size_t nxt = SIZE_MAX;
         for (size_t j = chain.back() + 1; j < pending.size() && nxt == SIZE_MAX; ++j)
           if (!gone[j] && pending[j].gemm.size() == 1 && !pending[j].side && chainable(*pending[j].gemm[0]) &&
@@ -1974,10 +1975,10 @@ void Executor::build() {
   {
     auto like = [](const GemmJob& x, const GemmJob& y) {
       const hk::GemmArgs &a = x.g, &b = y.g;
-      const int split = hk::gemm_split_for(a.m, a.n, a.k, a.defer, a.h16);
+      const int split = hk::gemm_split_for(a.m, a.n, a.k, a.defer, a.h16, false, a.on16);
       return a.m == b.m && a.n == b.n && a.k == b.k && a.lda == b.lda && a.ldb == b.ldb && a.ldc == b.ldc &&
              a.ta == b.ta && a.tb == b.tb && a.sum_a == b.sum_a && a.defer == b.defer && a.pad_a == b.pad_a &&
-             a.pad_b == b.pad_b && a.pad_c == b.pad_c && a.h16 == b.h16 && x.epi.act == y.epi.act &&
+             a.pad_b == b.pad_b && a.pad_c == b.pad_c && a.h16 == b.h16 && a.on16 == b.on16 && x.epi.act == y.epi.act &&
              (x.bias_id >= 0) == (y.bias_id >= 0) && (x.cs_id >= 0) == (y.cs_id >= 0) &&
              (x.epi.node != x.id) == (y.epi.node != y.id) && (x.ws != nullptr) == (y.ws != nullptr) &&
              (split == 1 || a.defer) && !x.ce_part && !x.ce_tab && !y.ce_part && !y.ce_tab && x.epi.drop < 0 &&
@@ -2048,17 +2049,13 @@ void Executor::build() {
   // writes no f32 value, and its readers get no f32 pointer for it, so that any other kernel
   // refuses the problem loudly.
   if (mixed_twins && !s_.opt_.plan_only) {
-    auto has16 = [&](uint32_t v) { return token16_.count(v) || fixed16_.count(v); };
     std::map<uint32_t, GemmJob*> job_of;   // MatMul node -> its GEMM job
     std::map<int64_t, GemmJob*> sums_of;  // fused SumRows node -> its GEMM job
     std::map<uint32_t, GemmJob*> producer;
     std::set<const GemmJob*> certain;     // jobs whose launch runs gemm16
     for (auto& pd : pending) {
       bool all = !pd.gemm.empty();
-      for (auto& j : pd.gemm) {
-        all = all && has16(j->asrc) && has16(j->bsrc) && hk::gemm16_fits(j->g);
-        for (auto& sg : j->segs) all = all && has16(sg.first) && has16(sg.second);
-      }
+      for (auto& j : pd.gemm) all = all && j->g.on16;
       for (auto& j : pd.gemm) {
         const Node& jn = p.node(j->id);
         job_of[jn.op == Op::AddRows ? jn.operands[0] : j->id] = j.get();

@@ -112,6 +112,8 @@ def mixed(ctx):
     (72, 1032, 88),     # 64 x 32 tiles, a K tail of 8
     (8, 256, 8),        # one partial tile
     (296, 9000, 200),   # split-K slices and their sum
+    (520, 2052, 260),   # rows of 4 mod 8 halves: the other kernel's 128 x 128 tiles, K in slices
+    (260, 1028, 516),   # the same, slices of 32 K and a K tail of 4
 ])
 def test_mixed_gemm_tiles(mixed, m, k, n, ta, tb):
     """Every tile of the f16 GEMM at partial tiles and K tails, against the float64 product of the
@@ -186,6 +188,28 @@ def test_mixed_chains_of_products(mixed, rows, h):
     for a, w in ((a1, w1), (a2, w2), (a3, w3)):
         want, mag = want + f16(a) @ f16(w).T, mag + np.abs(f16(a)) @ np.abs(f16(w)).T
     assert np.max(np.abs(got - want) / mag) <= 1e-5
+
+
+@pytest.mark.parametrize("rows,h", [(40, 512), (64, 1024), (16, 352), (2100, 512)])
+def test_chains_of_products_over_a_deep_k(ctx, rows, h):
+    """The same in f32 where the joined K would be split (1024 or more, few rows): the chain joins as
+    far as its product stays unsplit, against float64 (1e-5 of the sum of |terms|)."""
+    rng = np.random.default_rng(h + rows)
+    inputs = {"x": rng.standard_normal((rows, h)).astype(np.float32)}
+    p = Prog()
+    total = p.input("x", (rows, h))
+    want, mag = inputs["x"].astype(np.float64), np.abs(inputs["x"]).astype(np.float64)
+    for k in (1, 2, 3):
+        a, w = rng.standard_normal((rows, h)).astype(np.float32), rng.standard_normal((h, h)).astype(np.float32)
+        inputs.update({f"a{k}": a, f"w{k}": w})
+        ai, wi = p.input(f"a{k}", (rows, h)), p.input(f"w{k}", (h, h))
+        total = p.op("Add", [total, p.op("MatMul", [ai, p.op("Transpose", [wi], (h, h))], (rows, h))], (rows, h))
+        want = want + a.astype(np.float64) @ w.T
+        mag = mag + np.abs(a.astype(np.float64)) @ np.abs(w.T)
+    p.out(total)
+    prog = ctx.program(p.text())
+    prog.run(inputs)
+    assert np.max(np.abs(prog.output(0, rows * h).reshape(rows, h) - want) / mag) <= 1e-5
 
 
 @pytest.mark.parametrize("m,k,n,bias", [(70, 48, 30522, True), (4099, 32, 515, False), (37, 144, 60001, True), (2100, 16, 1001, False)])

@@ -177,3 +177,23 @@ def test_attention_row_counts_are_refused_by_the_plan(L, S, H, heads, taken):
             with pytest.raises(api.MsxError, match="no HIP kernel") as e:
                 forward_plan(p, False)
             assert e.value.code == -5, (op, e.value.code)
+
+
+@pytest.mark.parametrize("m,k,n,mixed,split", [
+    (4096, 5003, 256, True, 16),  # an untied head's input gradient over 5003 classes: 64 tiles of 128 x 128
+    (2016, 580, 192, True, 1),    # K under 1024: unsplit
+    (1000, 2052, 260, True, 22),  # rows of 4 mod 8 halves: 24 tiles, 22 slices of 96 K
+    (4096, 5008, 256, True, 1),   # whole 16-byte groups: gemm16, which has smaller tiles instead
+    (1000, 9000, 264, True, 4),   # the same with a deep K: 8 of its 256 x 192 tiles, slices of 2048 K or more
+])
+def test_a_product_is_split_for_the_kernel_that_runs_it(m, k, n, mixed, split):
+    """Split-K slices fill the chip with the tiles of the kernel that takes the product: 128 x 128 ones,
+    about 1024 blocks, for a mixed product whose pitches are no multiple of 8. The slices show in the
+    arena: m n floats each beside the operands, their f16 copies and the outputs."""
+    p = Prog()
+    a, b, bias = p.input("a", (m, k)), p.input("b", (k, n)), p.input("bias", (n,))
+    p.out(p.op("AddRows", [p.op("MatMul", [a, b], (m, n)), bias], (m, n)))
+    plan = forward_plan(p, mixed)
+    assert sum(l["what"].startswith("MatMul") for l in plan["launches"]) == 1
+    slices = (plan["arena"] - 6 * (m * k + k * n) - 4 * n) / (4 * m * n) - 1  # less the output itself
+    assert abs(slices - (split if split > 1 else 0)) <= 0.01, slices
