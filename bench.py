@@ -87,6 +87,16 @@ def measured_traffic(launch):
     return None
 
 
+def dispatch_places(rows, launch):
+    """Where a launch's dispatches sit among those of a profiled step (rocprofv3 counter runs). The
+    step's first dispatch copies its inputs, ahead of the launches the profile times."""
+    count = [len(kernels.split("+")) if kernels else 0 for _, _, _, _, kernels, _ in rows]
+    at = [what for what, *_ in rows].index(launch)
+    first = 1 + sum(n * runs for n, (*_, runs) in zip(count[:at], rows))
+    return {"step_dispatches": 1 + sum(n * runs for n, (*_, runs) in zip(count, rows)), "first": first,
+            "count": count[at]}
+
+
 def copy_once(ctx, mib):
     """One elementwise copy of `mib` MiB on the device (StopGradient: read n floats, write n)."""
     import numpy as np
@@ -199,14 +209,7 @@ def main():
             for what, ms, flop, nbytes, kernels, runs in rows:
                 f.write(json.dumps({"launch": what, "ms": ms, "flop": flop, "bytes": nbytes, "kernels": kernels,
                                     "runs": runs}) + "\n")
-    # Where the dominant launch's dispatches sit in a profiled step (rocprofv3 counter runs).
-    first = 0
-    for what, _, _, _, kernels, runs in rows:
-        if what == top["launch"]:
-            break
-        first += (len(kernels.split("+")) if kernels else 0) * runs
-    dispatches = {"step_dispatches": sum((len(r[4].split("+")) if r[4] else 0) * r[5] for r in rows), "first": first,
-                  "count": len(top["kernel"].split("+")) if top["kernel"] else 0}
+    dispatches = dispatch_places(rows, top["launch"])
     traffic = measured_traffic(top["launch"]) if args.config == "bert_tiny" else None
     stats = ctx.stats()
     ctx_scale = list(ctx.loss_scale()) if w["mixed"] else None
