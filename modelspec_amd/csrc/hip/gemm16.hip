@@ -42,6 +42,9 @@ namespace {
 template <int I, int J, bool AKC, bool BKC, int SA, int SB, int NA, int NB>
 __device__ __forceinline__ void read_frags(const uint32_t (&pa)[NA], const uint32_t (&pb)[NB], v8h (&fa)[I], v8h (&fb)[J]) {
 #if defined(__HIP_DEVICE_COMPILE__)
+  // The tiles and layouts written out below: any other would compile to no read at all.
+  static_assert((I == 8 && J == 3 && (AKC || !BKC)) || (I == 4 && J == 4) || (I == 2 && (J == 2 || J == 1)),
+                "no fragment reads for this tile and layout");
   [[maybe_unused]] v4s16 la[I], ha[I], lb[J], hb[J];
   if constexpr (I == 8 && J == 3 && AKC && BKC)
     asm volatile(
