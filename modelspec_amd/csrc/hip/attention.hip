@@ -11,6 +11,7 @@
 #include <cmath>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 
 #include "kernels.h"
 #include "device.h"
@@ -1264,15 +1265,18 @@ void launch_bwd(hipStream_t s, dim3 grid, unsigned qy, bool one, const float* q,
   MSX_LAUNCH((k_attn_bwd_mfma<D, T, W, KS>), grid, dim3(64 * W), lds, s, q, k, v, mask, o, stats, g, dq, dk, dv, L, S,
              H, heads, scale, int(qy));
 }
-// Dispatch on a plan: the f16 kernels (never split) or the f32 ones.
+// Dispatch on a plan, within a template on D: the f16 kernels (never split) or the f32 ones, those that
+// attn_plan gives heads of this width.
 #define MSX_BY_PLAN(plan, h16, GO_H, GO_F)                 \
   if (h16) {                                               \
     if ((plan).W == 4) GO_H(32, 4);                        \
-    else if ((plan).T == 64) GO_H(64, 2);                  \
+    else if constexpr (D <= 64) GO_H(64, 2);               \
     else GO_H(32, 2);                                      \
   } else {                                                 \
-    if ((plan).KS == 2) GO_F(128, 4, 2);                   \
-    else if ((plan).W == 4) GO_F(32, 4, 1);                \
+    if constexpr (D <= 64) {                               \
+      if ((plan).KS == 2) GO_F(128, 4, 2);                 \
+      else GO_F(32, 4, 1);                                 \
+    } else if ((plan).W == 4) GO_F(32, 4, 1);              \
     else GO_F(32, 2, 1);                                   \
   }
 }  // namespace
@@ -1282,13 +1286,16 @@ bool attention_fits(int64_t l, int64_t s, int64_t d, bool gradient) {
   return head_ok(d) && s <= 65535 && bwd_fits(s, s, d) && (gradient ? bwd_fits(l, s, d) : fwd_fits(l, s, d));
 }
 
-#define MSX_BY_D(d, call)                          \
-  switch (d) {                                     \
-    case 16: call(16); break;                      \
-    case 32: call(32); break;                      \
-    case 64: call(64); break;                      \
-    default: call(128); break;                     \
+// go(integral_constant of the head width).
+template <class Go>
+void by_width(int64_t d, Go&& go) {
+  switch (d) {
+    case 16: go(std::integral_constant<int, 16>{}); break;
+    case 32: go(std::integral_constant<int, 32>{}); break;
+    case 64: go(std::integral_constant<int, 64>{}); break;
+    default: go(std::integral_constant<int, 128>{}); break;
   }
+}
 
 void attention_fwd(hipStream_t s, const float* q, const float* k, const float* v, const float* mask, float* o,
                    float* stats, int64_t B, int64_t L, int64_t S, int64_t H, int64_t heads, bool h16, _Float16* o16) {
@@ -1312,14 +1319,16 @@ void attention_fwd(hipStream_t s, const float* q, const float* k, const float* v
 #define GO_H(T, W) launch_fwd_h<D, T, W>(s, grid, q, k, v, mask, o, stats, int(L), int(S), int(H), int(heads), scale, o16)
 #define GO_F(T, W, KS) \
   launch_fwd<D, T, W, KS>(s, grid, plan.one, q, k, v, mask, o, stats, int(L), int(S), int(H), int(heads), scale)
-#define GO(D_)                                                 \
-  {                                                            \
-    constexpr int D = D_;                                      \
-    if (D <= 64 && plan.T == 64 && plan.KS == 2) GO_F(64, 4, 2); \
-    else MSX_BY_PLAN(plan, h16, GO_H, GO_F)                    \
-  }
-  MSX_BY_D(d, GO)
-#undef GO
+  by_width(d, [&](auto width) {
+    constexpr int D = decltype(width)::value;
+    if constexpr (D <= 64) {
+      if (plan.T == 64 && plan.KS == 2) {
+        GO_F(64, 4, 2);
+        return;
+      }
+    }
+    MSX_BY_PLAN(plan, h16, GO_H, GO_F)
+  });
 #undef GO_F
 #undef GO_H
 }
@@ -1344,9 +1353,10 @@ void attention_bwd(hipStream_t s, const float* q, const float* k, const float* v
 #define GO_F(T, W, KS)                                                                                              \
   launch_bwd<D, T, W, KS>(s, gb, row_blocks(L, pq), pq.one, q, k, v, mask, o, stats, g, dq, dk, dv, int(L), int(S), \
                         int(H), int(heads), scale)
-#define GO(D_) { constexpr int D = D_; MSX_BY_PLAN(pq, false, GO_H, GO_F) }
-    MSX_BY_D(d, GO)
-#undef GO
+    by_width(d, [&](auto width) {
+      constexpr int D = decltype(width)::value;
+      MSX_BY_PLAN(pq, false, GO_H, GO_F)
+    });
 #undef GO_F
 #undef GO_H
     return;
@@ -1356,9 +1366,10 @@ void attention_bwd(hipStream_t s, const float* q, const float* k, const float* v
 #define GO_F(T, W, KS)                                                                                            \
   launch_bwd_q<D, T, W, KS>(s, gq, pq.one, q, k, v, mask, o, stats, g, dq, dsum, int(L), int(S), int(H), int(heads), \
                           scale)
-#define GO(D_) { constexpr int D = D_; MSX_BY_PLAN(pq, h16, GO_H, GO_F) }
-  MSX_BY_D(d, GO)
-#undef GO
+  by_width(d, [&](auto width) {
+    constexpr int D = decltype(width)::value;
+    MSX_BY_PLAN(pq, h16, GO_H, GO_F)
+  });
 #undef GO_F
 #undef GO_H
   if (dk || dv) {
@@ -1370,37 +1381,35 @@ void attention_bwd(hipStream_t s, const float* q, const float* k, const float* v
 #define GO_F(T, W, KS)                                                                                             \
   launch_bwd_kv<D, T, W, KS>(s, gk, pk.one, q, k, v, mask, stats, g, dsum, dk, dv, int(L), int(S), int(H), int(heads), \
                            scale)
-#define GO(D_) { constexpr int D = D_; MSX_BY_PLAN(pk, h16, GO_H, GO_F) }
-    MSX_BY_D(d, GO)
-#undef GO
+    by_width(d, [&](auto width) {
+      constexpr int D = decltype(width)::value;
+      MSX_BY_PLAN(pk, h16, GO_H, GO_F)
+    });
 #undef GO_F
 #undef GO_H
   }
 }
 
 void prepare_attention() {
+  // Every kernel that a launch above reaches.
   const void* kernels[] = {
-#define MSX_ATTN_W(D, T, W)                                         \
-  reinterpret_cast<const void*>(k_attn_fwd_mfma<D, T, W>),          \
-      reinterpret_cast<const void*>(k_attn_fwd_mfma<D, 64, 4, 2>),  \
-      reinterpret_cast<const void*>(k_attn_bwd_q_mfma<D, T, W>),    \
-      reinterpret_cast<const void*>(k_attn_bwd_kv_mfma<D, T, W>),   \
-      reinterpret_cast<const void*>(k_attn_fwd_mfma<D, 128, 4, 2>), \
-      reinterpret_cast<const void*>(k_attn_bwd_q_mfma<D, 128, 4, 2>), \
-      reinterpret_cast<const void*>(k_attn_bwd_kv_mfma<D, 128, 4, 2>), \
-      reinterpret_cast<const void*>(k_attn_bwd_mfma<D, T, W>),      \
-      reinterpret_cast<const void*>(k_attn_bwd_mfma<D, 128, 4, 2>)
+#define MSX_ATTN_F(D, T, W, KS)                                     \
+  reinterpret_cast<const void*>(k_attn_fwd_mfma<D, T, W, KS>),      \
+      reinterpret_cast<const void*>(k_attn_bwd_q_mfma<D, T, W, KS>), \
+      reinterpret_cast<const void*>(k_attn_bwd_kv_mfma<D, T, W, KS>), \
+      reinterpret_cast<const void*>(k_attn_bwd_mfma<D, T, W, KS>)
 #define MSX_ATTN_H(D, T, W)                                         \
   reinterpret_cast<const void*>(k_attn_fwd_h16<D, T, W>),           \
       reinterpret_cast<const void*>(k_attn_bwd_q_h16<D, T, W>),     \
       reinterpret_cast<const void*>(k_attn_bwd_kv_h16<D, T, W>)
-#define MSX_ATTN_K(D)                                                                            \
-  MSX_ATTN_W(D, 32, 4), MSX_ATTN_W(D, 32, 2), MSX_ATTN_H(D, 32, 4), \
-      MSX_ATTN_H(D, 64, 2), MSX_ATTN_H(D, 32, 2)
-      MSX_ATTN_K(16), MSX_ATTN_K(32), MSX_ATTN_K(64), MSX_ATTN_K(128)};
+#define MSX_ATTN_K(D)                                                           \
+  MSX_ATTN_F(D, 32, 4, 1), MSX_ATTN_F(D, 128, 4, 2), MSX_ATTN_H(D, 32, 4),       \
+      MSX_ATTN_H(D, 64, 2), reinterpret_cast<const void*>(k_attn_fwd_mfma<D, 64, 4, 2>)
+      MSX_ATTN_K(16), MSX_ATTN_K(32), MSX_ATTN_K(64),
+      MSX_ATTN_F(128, 32, 4, 1), MSX_ATTN_F(128, 32, 2, 1), MSX_ATTN_H(128, 32, 4), MSX_ATTN_H(128, 32, 2)};
 #undef MSX_ATTN_K
 #undef MSX_ATTN_H
-#undef MSX_ATTN_W
+#undef MSX_ATTN_F
   for (const void* kern : kernels) {
     hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(kLdsMax));
     if (e != hipSuccess) throw std::runtime_error(std::string("hipFuncSetAttribute: ") + hipGetErrorString(e));
