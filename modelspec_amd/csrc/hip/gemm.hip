@@ -666,19 +666,14 @@ void gemm_group(hipStream_t s, const GemmArgs* list, int count) {
   if (plan.wm == 2) MSX_WIDE(TA, TB, 2, 2, 16);             \
   else if (plan.wn == 2) MSX_WIDE(TA, TB, 1, 2, 16);        \
   else MSX_WIDE(TA, TB, 1, 1, 32);
-  // The mixed-precision variants: the same tiles with f16 K tiles of 32.
-#define MSX_WIDE_HV(TA, TB, WM, WN, VA, VB)                                                                 \
-  MSX_LAUNCH((k_gemm_w<TA, TB, WM, WN, 32, VA, VB, true>), wgrid, dim3(256), 0, s, ptrs, g.m, g.n, g.k,     \
+  // The mixed-precision variants: 128 x 128 tiles with f16 K tiles of 32.
+#define MSX_WIDE_HV(TA, TB, VA, VB)                                                                         \
+  MSX_LAUNCH((k_gemm_w<TA, TB, 4, 4, 32, VA, VB, true>), wgrid, dim3(256), 0, s, ptrs, g.m, g.n, g.k,       \
              g.lda, g.ldb, g.ldc, chunk, g.sum_a, vo, order)
-#define MSX_WIDE_H(TA, TB, WM, WN)                                  \
-  if (va && vb) MSX_WIDE_HV(TA, TB, WM, WN, true, true);            \
-  else if (vb) MSX_WIDE_HV(TA, TB, WM, WN, false, true);            \
-  else MSX_WIDE_HV(TA, TB, WM, WN, false, false)
 #define MSX_WIDE_HT(TA, TB)                                 \
-  if (plan.wm == 4) MSX_WIDE_H(TA, TB, 4, 4);               \
-  else if (plan.wm == 2) MSX_WIDE_H(TA, TB, 2, 2);          \
-  else if (plan.wn == 2) MSX_WIDE_H(TA, TB, 1, 2);          \
-  else MSX_WIDE_H(TA, TB, 1, 1);
+  if (va && vb) MSX_WIDE_HV(TA, TB, true, true);            \
+  else if (vb) MSX_WIDE_HV(TA, TB, false, true);            \
+  else MSX_WIDE_HV(TA, TB, false, false)
   // The cross-entropy head kernels: the largest tile of each precision, both operands float4.
 #define MSX_CE_V(TA, TB, WM, WN, WK, H, CE)                                                                    \
   MSX_LAUNCH((k_gemm_w<TA, TB, WM, WN, WK, true, true, H, CE>), wgrid, dim3(256), 0, s, ptrs, g.m, g.n, g.k,  \
@@ -724,10 +719,10 @@ void gemm_group(hipStream_t s, const GemmArgs* list, int count) {
     else { MSX_CE(2, 2, 16, false) }
   } else if (g.h16) {
     if (g.colsum) bad("mixed-precision column sums need gemm16's layout (f16 copies, rows of whole 16-byte groups)");
-    if (!g.ta && !g.tb) { MSX_WIDE_HT(false, false) }
-    else if (g.ta && !g.tb) { MSX_WIDE_HT(true, false) }
-    else if (!g.ta && g.tb) { MSX_WIDE_HT(false, true) }
-    else { MSX_WIDE_HT(true, true) }
+    if (!g.ta && !g.tb) { MSX_WIDE_HT(false, false); }
+    else if (g.ta && !g.tb) { MSX_WIDE_HT(true, false); }
+    else if (!g.ta && g.tb) { MSX_WIDE_HT(false, true); }
+    else { MSX_WIDE_HT(true, true); }
   } else if (!g.ta && !g.tb) { MSX_WIDE_T(false, false) }
   else if (g.ta && !g.tb) { MSX_WIDE_T(true, false) }
   else if (!g.ta && g.tb) { MSX_WIDE_T(false, true) }
@@ -738,7 +733,6 @@ void gemm_group(hipStream_t s, const GemmArgs* list, int count) {
 #undef MSX_CE_T
 #undef MSX_CE_V
 #undef MSX_WIDE_HT
-#undef MSX_WIDE_H
 #undef MSX_WIDE_HV
 #undef MSX_WIDE_T
 #undef MSX_WIDE
