@@ -1,5 +1,5 @@
-"""Benchmark of the BERT-tiny masked-LM training step on one MI355X;
-with `--config bert_base`, of the BERT-base mixed-precision step.
+"""Benchmark of the BERT-tiny masked-LM training step on one MI355X; with `--config bert_base`, of
+the BERT-base mixed-precision step.
 
 One step = forward + backward + AdamW of BERT-tiny (2 layers, hidden 128, 2 heads, FFN 512,
 V = 30522, batch 32, seq 128, dropout 0.1, the masked-row gather of 832 rows) on synthetic Zipf

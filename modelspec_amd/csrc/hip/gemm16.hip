@@ -18,7 +18,8 @@ namespace msx::hk {
 // Both XORs are laid out for the lane groups the LDS serves together: a ds_read_b128 takes lanes 0-3,
 // 12-15, 20-27 in one pass and 4-11, 16-19, 28-31 in the next (and so for lanes 32-63), a transposed
 // read lanes 0-31 and 32-63. With the slots spread over 16 consecutive lanes instead, half of the LDS
-// cycles were bank conflicts (SQ_LDS_BANK_CONFLICT / SQ_LDS_IDX_ACTIVE 0.50, now 0.01).
+// cycles were bank conflicts (SQ_LDS_BANK_CONFLICT / SQ_LDS_IDX_ACTIVE over BERT-base's step 0.50, now
+// 0.03 to 0.06, the output's way through LDS included).
 // BK 64 loads whole 128-byte lines of a KC operand: the loads alone of 16384 x 768 x 3072 take 56 us
 // against 71 with 64-byte rows (BK 32).
 //

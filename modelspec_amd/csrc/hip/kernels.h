@@ -239,18 +239,17 @@ void dropout(hipStream_t s, const float* x, float* o, int64_t n, const int32_t* 
 // Attention over a key mask [B, S]; q [B*L, H], k/v [B*S, H] (attention.hip).
 // Whether a launch takes these row counts and head width (l query rows, s key rows a sequence).
 bool attention_fits(int64_t l, int64_t s, int64_t d, bool gradient);
-
 // stats: [B*heads*L, 2] softmax maximum and sum per query (written when non-null; required by the
-// MFMA backward).
-// h16 (mixed precision): the MFMA path's contractions on the f16 MFMA with f32 accumulation.
+// backward).
+// h16 (mixed precision): the contractions on the f16 MFMA with f32 accumulation, where attention_f16.
 void attention_fwd(hipStream_t s, const float* q, const float* k, const float* v, const float* mask, float* o,
                    float* stats, int64_t B, int64_t L, int64_t S, int64_t H, int64_t heads, bool h16 = false,
                    _Float16* o16 = nullptr);
 // Whether h16 attention of these row counts runs in f16; its kernels then also write f16 copies of
 // their outputs where asked (o16; dq16, dk16, dv16).
 bool attention_f16(int64_t l, int64_t s);
-// Any of dk/dv may be null; the MFMA path needs dq, o (the forward's output), stats and dsum
-// ([B*heads*L] scratch).
+// Any of dk/dv may be null; dq, o (the forward's output), stats and dsum ([B*heads*L] scratch) are
+// needed.
 void attention_bwd(hipStream_t s, const float* q, const float* k, const float* v, const float* mask, const float* o,
                    const float* stats, const float* g, float* dq, float* dk, float* dv, float* dsum, int64_t B,
                    int64_t L, int64_t S, int64_t H, int64_t heads, bool h16 = false, _Float16* dq16 = nullptr,

@@ -1,6 +1,6 @@
-"""Full-length runs of the BASELINE configs on the MI355X against the CPU oracle's runs of the same
+"""Full-length parity runs on the MI355X against the CPU oracle's runs of the same
 seed and inputs: the MLP classifier for 1,000 steps, the transformer block for 500 and BERT-tiny
-for 1,000 ("Parity runs"). The oracle takes minutes to hours for them on one core, so
+for 1,000. The oracle takes minutes to hours for them on one core, so
 its runs are fixtures (tests/golden/oracle_*_<config>_<steps>.*): every loss, and every parameter
 element (the MLP) or a seeded sample of at least 65,536 elements stratified over every tensor (the
 transformer block, BERT-tiny), is held to the reference's run tolerance, and every tensor of the

@@ -60,7 +60,7 @@ def test_linear_regression_is_bit_identical_to_the_golden_run(ctx, oracle):
 
 
 def test_linear_regression_on_the_baseline_distribution(ctx, oracle):
-    """BASELINE configs[0] as stated there: x ~ U(-1, 1) [8, 4], w_true ~ U(-1, 1) [4, 1] and
+    """The linear regression on its noisy distribution: x ~ U(-1, 1) [8, 4], w_true ~ U(-1, 1) [4, 1] and
     y = x w_true + N(0, 0.01) noise (standard deviation 0.01), a fresh batch each step, SGD lr 0.1
     for 500 steps from the seed-42 xavier initialisation. The same step program and inputs go to
     the oracle one step at a time (its printed step program: loss, gradient and updated weight);
