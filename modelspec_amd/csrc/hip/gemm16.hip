@@ -203,7 +203,9 @@ __device__ __forceinline__ void read_frags(const uint32_t (&pa)[NA], const uint3
 #undef MSX_RWAIT
 
 // GELU and its gradient for values that leave as f16: x s and g (s + x s'), s = 1 / (1 + exp(-v)),
-// v = 2 sqrt(2/pi) (x + 0.044715 x^3), on the hardware exp2 and reciprocal (1 ulp each).
+// v = 2 sqrt(2/pi) (x + 0.044715 x^3), on the hardware exp2 and reciprocal (1 ulp each). Against 64 bits
+// over x of N(0, 1): 4.7e-8 and 6.6e-8 in f32, where d_gelu and d_gelu_grad have 4.6e-8 and 5.7e-8; rounded
+// to f16 2.0649e-4 and 2.0755e-4 with either.
 constexpr float kGeluA = -2.0f * 0.797884560802865f * 1.4426950408889634f, kGeluB = kGeluA * 0.044715f;
 __device__ __forceinline__ float gelu16(float x) {
   const float e = __builtin_amdgcn_exp2f(x * __builtin_fmaf(kGeluB, x * x, kGeluA));  // exp(-v)
